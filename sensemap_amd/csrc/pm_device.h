@@ -18,6 +18,10 @@ constexpr int kQuadPad = 4;          // zero texels around every source image
 // Shapes: lw = 4 (16x32), 5 (32x16, the default), 6 (64x8).
 constexpr int kTileLog2WMin = 4, kTileLog2WMax = 6, kTileLog2WDefault = 5;
 constexpr int kTilePixels = 512;
+constexpr int kTileLog2Px = 8;       // pixels of one colour in a tile: 256
+// The sweep and the local optimisation can also run on tiles of 16x8 pixels,
+// 64 of a colour, whose evaluations the workgroup's four waves share.
+constexpr int kSmallTileLog2W = 4, kSmallTileLog2Px = 6;
 constexpr int kMaxBlocksPerCU = 8;   // resident workgroups of a persistent launch per CU, at most
 constexpr int kSweepThreads = 256;
 constexpr float kMaxCost = 2.0f;
@@ -70,13 +74,12 @@ struct ViewDev {
   SrcDev src[PM_MAX_NUM_SRC];
 };
 
-// Workspace fields per thread of a launch (SoA over the launch's threads:
-// field f of slot s at ws[f * ws_slots + s], ws_slots = blocks * 256).
+// Workspace floats per pixel of a tile:
 //   hyp   : 4 * (kMaxHyp + kNumRefine) floats  (nx, ny, nz, d per hypothesis)
 //   M     : kMaxHyp * N floats      (candidate x source costs)
 //   RM    : kNumRefine * N floats   (refinement x source costs)
 //   W     : N floats                (view weights, later CDF)
-inline int ws_floats_per_slot(int N) {
+inline int ws_floats_per_pixel(int N) {
   return 4 * (kMaxHyp + kNumRefine) + kMaxHyp * N + kNumRefine * N + N;
 }
 
@@ -92,14 +95,16 @@ struct LaunchEntry {
 };
 
 // A launch runs `grid` persistent workgroups over `total_tiles` tiles.  Each
-// workgroup owns 256 workspace slots (one per thread) for the whole launch,
-// so no two resident workgroups ever share workspace lines, and the launch
-// boundary makes the workspace coherent across the XCDs' L2 caches.
+// workgroup owns ws_stride floats of workspace (its tile's pixels) for the
+// whole launch, so no two resident workgroups ever share workspace lines, and
+// the launch boundary makes the workspace coherent across the XCDs' L2 caches.
 struct LaunchTable {
   int32_t n;             // entries
   int32_t total_tiles;   // tiles of the launch
-  int32_t ws_slots;      // grid * 256
+  int32_t ws_stride;     // workspace floats per workgroup
   int32_t tile_lw;       // log2 of the tile width (kTileLog2WMin..kTileLog2WMax)
+  int32_t tile_lpx;      // log2 of a tile's pixels of one colour (kTileLog2Px or kSmallTileLog2Px)
+  int32_t pad0;
   float* ws;             // workspace of the launch
   uint32_t* queue;       // 8 tile counters (one per XCD range), zero at launch start
   LaunchEntry e[1];      // n entries follow (allocated with the table)
@@ -109,10 +114,10 @@ inline size_t launch_table_bytes(int n) {
   return sizeof(LaunchTable) + (size_t)(n > 1 ? n - 1 : 0) * sizeof(LaunchEntry);
 }
 
-// Tiles of a view at tile width 2^lw (one workgroup iteration each per
-// colour pass).
-inline int view_tiles(int W, int H, int lw) {
-  const int tw = 1 << lw, th = kTilePixels >> lw;
+// Tiles of a view at tile width 2^lw and 2^lpx pixels of a colour per tile
+// (one workgroup iteration each per colour pass).
+inline int view_tiles(int W, int H, int lw, int lpx) {
+  const int tw = 1 << lw, th = (2 << lpx) >> lw;
   return ((W + tw - 1) / tw) * ((H + th - 1) / th);
 }
 
@@ -136,7 +141,7 @@ hipError_t launch_ref_moments(const ViewDev* v, int W, int H, int accum_mode, fl
                               uint8_t* grad_ok, hipStream_t s);
 // Table-driven colour-pass launches: `table` is a device copy of a
 // LaunchTable whose queue counters are zero; `grid` comes from phase_grid
-// for the table's total_tiles (and sized its ws_slots).
+// for the table's total_tiles.
 enum PhaseKind {
   kPhaseInit = 0,
   kPhaseSweep = 1,
@@ -153,6 +158,8 @@ inline bool plain_phase(PhaseKind k) { return k >= kPhaseFilter; }
 // number of CUs times the workgroups one CU holds (capped by blocks_per_cu
 // when > 0), and never more than the tiles.
 int phase_grid(PhaseKind kind, const LaunchCfg& cfg, int tiles, int blocks_per_cu);
+// Whether a launch that would have `tiles` tiles of 256 pixels runs on tiles of 64.
+bool small_tiles(PhaseKind kind, const LaunchCfg& cfg, int tiles, int blocks_per_cu);
 // Workgroups of the phase kernel one CU holds at once.
 int phase_occupancy(PhaseKind kind, const LaunchCfg& cfg);
 hipError_t launch_phase(PhaseKind kind, const LaunchCfg& cfg, const LaunchTable* table, int grid, hipStream_t s);

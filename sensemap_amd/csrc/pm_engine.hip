@@ -886,8 +886,24 @@ pm_status plan_launches(const std::vector<std::pair<pm_problem*, const std::vect
     pm::LaunchCfg cfg;
     pm_tuning shape;
     std::vector<pm::LaunchEntry> e;
+    std::vector<const pm_problem*> views;  // of the entries
     int tiles = 0;
     int nmax = 1;  // most sources of a view in the launch (workspace size)
+    int lw = 0, lpx = pm::kTileLog2Px;
+
+    // Number the tiles of width 2^w with 2^px pixels of a colour.
+    pm_status number_tiles(int w, int px) {
+      lw = w;
+      lpx = px;
+      long long n = 0;
+      for (size_t k = 0; k < e.size(); ++k) {
+        e[k].tile_start = (int32_t)n;
+        n += pm::view_tiles(views[k]->W, views[k]->H, w, px);
+        if (n > INT32_MAX) return fail(PM_ERR_INVALID_ARG, "too many tiles in one launch");
+      }
+      tiles = (int)n;
+      return PM_OK;
+    }
   };
   std::vector<Group> groups;
   for (const auto& ph : phases) {
@@ -901,23 +917,25 @@ pm_status plan_launches(const std::vector<std::pair<pm_problem*, const std::vect
             gg.shape.blocks_per_cu == shape.blocks_per_cu)
           g = &gg;
       if (!g) {
-        groups.push_back(Group{r.kind, cfg, shape, {}, 0, 1});
+        groups.push_back(Group{r.kind, cfg, shape, {}, {}, 0, 1});
         g = &groups.back();
       }
       pm::LaunchEntry en{};
       en.v = p->dev;
-      en.tile_start = g->tiles;
       en.color = r.color;
       en.pass = r.pass;
       en.th_mc = r.th_mc;
       g->e.push_back(en);
-      const long long tiles = (long long)g->tiles + pm::view_tiles(p->W, p->H, g->shape.tile_lw);
-      if (tiles > INT32_MAX) return fail(PM_ERR_INVALID_ARG, "too many tiles in one launch");
-      g->tiles = (int)tiles;
+      g->views.push_back(p);
       g->nmax = std::max(g->nmax, p->N);
     }
   }
   for (Group& g : groups) {
+    pm_status rs = g.number_tiles(g.shape.tile_lw, pm::kTileLog2Px);
+    if (rs != PM_OK) return rs;
+    if (pm::small_tiles(g.kind, g.cfg, g.tiles, g.shape.blocks_per_cu)) {
+      if ((rs = g.number_tiles(pm::kSmallTileLog2W, pm::kSmallTileLog2Px)) != PM_OK) return rs;
+    }
     const int grid = pm::phase_grid(g.kind, g.cfg, g.tiles, g.shape.blocks_per_cu);
     if (grid <= 0) return fail(PM_ERR_DEVICE, "no launch configuration for a phase kernel");
     const size_t off = (plan.tables.size() + 15) & ~(size_t)15;
@@ -925,13 +943,14 @@ pm_status plan_launches(const std::vector<std::pair<pm_problem*, const std::vect
     pm::LaunchTable* lt = (pm::LaunchTable*)(plan.tables.data() + off);
     lt->n = (int32_t)g.e.size();
     lt->total_tiles = g.tiles;
-    lt->ws_slots = grid * pm::kSweepThreads;
-    lt->tile_lw = g.shape.tile_lw;
+    lt->ws_stride = pm::plain_phase(g.kind) ? 0 : pm::ws_floats_per_pixel(g.nmax) << g.lpx;
+    lt->tile_lw = g.lw;
+    lt->tile_lpx = g.lpx;
     lt->ws = nullptr;
     lt->queue = nullptr;
     std::memcpy(lt->e, g.e.data(), g.e.size() * sizeof(pm::LaunchEntry));
     plan.launches.push_back(pm_schedule::Launch{g.kind, g.cfg, off, g.tiles, grid});
-    plan.ws_floats = std::max(plan.ws_floats, (size_t)lt->ws_slots * pm::ws_floats_per_slot(g.nmax));
+    plan.ws_floats = std::max(plan.ws_floats, (size_t)grid * lt->ws_stride);
   }
   return PM_OK;
 }

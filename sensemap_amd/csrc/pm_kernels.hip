@@ -1,9 +1,11 @@
 // pm_kernels.hip -- gfx950 kernels of the PatchMatch MVS engine.
 //
-// One thread per pixel of one checkerboard colour.  A 256-thread workgroup
-// owns a 32x16 pixel tile (its 256 pixels of the colour); each wave64 covers
-// 4 rows x 16 same-colour pixels, so the 64 windows of a wave overlap and
-// their source footprints hit the same cache lines.  Per workgroup the
+// A 256-thread workgroup owns a 32x16 pixel tile (its 256 pixels of one
+// checkerboard colour), or a 16x8 one in small launches.  The sweep and the
+// local optimisation list the (hypothesis, pixel) pairs that need a cost and
+// walk the windows of 64 pairs per wave; neighbouring pairs are neighbouring
+// pixels, so the windows of a wave overlap and their source footprints hit
+// the same cache lines.  Per workgroup the
 // reference tile (+ window halo; one 32-bit word per texel holding the
 // intensity and 3x the intensity, see ncc_eval) and the 256-entry bilateral colour
 // table are staged in LDS; the spatial weight table and the per-source pose
@@ -37,6 +39,7 @@
 
 #include <map>
 #include <mutex>
+#include <utility>
 
 #include "pm_device.h"
 #include "pm_math.h"
@@ -92,19 +95,22 @@ struct Pix {
   bool shifted;          // compensated moments for this pixel
 };
 
-// Workspace accessors (SoA over slots).
+// Workspace of one workgroup: a contiguous region of the launch's workspace
+// holding, per pixel of a tile, hypotheses and costs ([field][pixel], so the
+// pixels of a wave read consecutive words).  npx pixels per tile.
 struct Ws {
   float* base;
-  int slots, slot, N;  // base/slots: the launch's workspace; slot: this thread
-  __device__ __attribute__((address_space(1))) float& hyp(int k, int c) const { return G(base)[(size_t)(4 * k + c) * slots + slot]; }
-  __device__ __attribute__((address_space(1))) float& M(int k, int i) const {
-    return G(base)[(size_t)(4 * (kMaxHyp + kNumRefine) + k * N + i) * slots + slot];
+  int npx, N;
+  __device__ __attribute__((address_space(1))) f4v& hyp(int k, int px) const {
+    return ((__attribute__((address_space(1))) f4v*)G(base))[k * npx + px];
   }
-  __device__ __attribute__((address_space(1))) float& RM(int k, int i) const {
-    return G(base)[(size_t)(4 * (kMaxHyp + kNumRefine) + kMaxHyp * N + k * N + i) * slots + slot];
+  __device__ __attribute__((address_space(1))) float& at(int row, int px) const {
+    return G(base)[4 * (kMaxHyp + kNumRefine) * npx + row * npx + px];
   }
-  __device__ __attribute__((address_space(1))) float& Wt(int i) const {
-    return G(base)[(size_t)(4 * (kMaxHyp + kNumRefine) + (kMaxHyp + kNumRefine) * N + i) * slots + slot];
+  __device__ __attribute__((address_space(1))) float& M(int k, int i, int px) const { return at(k * N + i, px); }
+  __device__ __attribute__((address_space(1))) float& RM(int k, int i, int px) const { return at((kMaxHyp + k) * N + i, px); }
+  __device__ __attribute__((address_space(1))) float& Wt(int i, int px) const {
+    return at((kMaxHyp + kNumRefine) * N + i, px);
   }
 };
 
@@ -653,8 +659,8 @@ struct Ctx {
   float th_mc;
   int local_block;  // tile index within the view
   int lw;           // log2 of the tile width
-  float* ws;
-  int ws_slots;
+  int lpx;          // log2 of the tile's pixels of one colour
+  float* ws;        // this workgroup's workspace
 };
 
 __device__ __forceinline__ Ctx resolve(const LaunchTable* __restrict__ lt, int t) {
@@ -672,16 +678,24 @@ __device__ __forceinline__ Ctx resolve(const LaunchTable* __restrict__ lt, int t
   c.th_mc = g->e[lo].th_mc;
   c.local_block = t - g->e[lo].tile_start;
   c.lw = g->tile_lw;
-  c.ws = g->ws;
-  c.ws_slots = g->ws_slots;
+  c.lpx = g->tile_lpx;
+  c.ws = g->ws + (size_t)blockIdx.x * g->ws_stride;
   return c;
 }
 
+// Where a tile lies, and its pixels of one colour.
+struct Geo {
+  int row0, col0, lw, color, pitch;
+  // Pixel px of the tile: 2^(lw-1) pixels of the colour per row.
+  __device__ __forceinline__ void pixel(int px, int& lrow, int& lcol) const {
+    lrow = px >> (lw - 1);
+    lcol = 2 * (px & ((1 << (lw - 1)) - 1)) + ((row0 + lrow + color) & 1);
+  }
+};
+
 // Stage the colour table, the spatial weights and the ref tile (zero outside
-// the image) into LDS, then map the thread to its pixel.  Returns false for
-// threads whose pixel lies outside the image (after the barrier).
-__device__ __forceinline__ bool setup_pass(const Ctx& cx, int R, int pitch, uint32_t* tile, float* ct, float* spl,
-                                           Pix& px) {
+// the image) into LDS.  The caller's barrier makes them visible.
+__device__ __forceinline__ Geo stage_tile(const Ctx& cx, int R, int pitch, uint32_t* tile, float* ct, float* spl) {
   const VPtr v = cx.v;
   const int t = threadIdx.x;
   ct[t] = G(v->ct)[t];
@@ -689,56 +703,96 @@ __device__ __forceinline__ bool setup_pass(const Ctx& cx, int R, int pitch, uint
   for (int e = t; e < nsp; e += kSweepThreads) spl[e] = G(v->sp)[e];
   const int W = v->W, H = v->H;
   const int lw = cx.lw;
+  const int rows = (2 << cx.lpx) >> lw;
   const int tiles_x = (W + (1 << lw) - 1) >> lw;
   const int ty = cx.local_block / tiles_x;
   const int tx = cx.local_block - ty * tiles_x;
-  const int row0 = ty * (kTilePixels >> lw), col0 = tx << lw;
+  const int row0 = ty * rows, col0 = tx << lw;
   const int tw = (1 << lw) + 2 * R;
-  const int th = (kTilePixels >> lw) + 2 * R;
+  const int th = rows + 2 * R;
   for (int e = t; e < tw * th; e += kSweepThreads) {
     const int er = e / tw, ec = e - er * tw;
     const int rr = row0 - R + er, cc = col0 - R + ec;
     const uint32_t ri = (rr < 0 || rr >= H || cc < 0 || cc >= W) ? 0u : (uint32_t)G(v->ref)[rr * W + cc];
     tile[er * pitch + ec] = (ri << 16) | (3u * ri);
   }
-  __syncthreads();
-  px.lrow = t >> (lw - 1);
-  px.row = row0 + px.lrow;
-  px.lcol = 2 * (t & ((1 << (lw - 1)) - 1)) + ((px.row + cx.color) & 1);
-  px.col = col0 + px.lcol;
-  if (px.row >= H || px.col >= W) return false;
-  px.p = px.row * W + px.col;
-  const f4v m = ld_f4(v->refm, px.p);
+  return Geo{row0, col0, lw, cx.color, pitch};
+}
+
+// The context of pixel (row, col) at tile position (lrow, lcol), with its
+// moments m.
+__device__ __forceinline__ Pix make_pix(VPtr v, const Geo& g, const uint32_t* tile, int R, int lrow, int lcol, f4v m) {
+  Pix px;
+  px.lrow = lrow;
+  px.lcol = lcol;
+  px.row = g.row0 + lrow;
+  px.col = g.col0 + lcol;
+  px.p = px.row * v->W + px.col;
   px.mu_r = m.x;
   px.var_r = m.y;
   px.inv_sw = m.z;
   px.err_r = m.w;
-  px.c = (int)(tile[(px.lrow + R) * pitch + px.lcol + R] >> 16);
+  px.c = (int)(tile[(lrow + R) * g.pitch + lcol + R] >> 16);
   px.shifted = (v->accum_mode == PM_ACCUM_COMPENSATED) && (px.var_r < kLowTexVar);
   px.np0 = v->refInvK[0] * (float)px.col + v->refInvK[1];
   px.np1 = v->refInvK[2] * (float)px.row + v->refInvK[3];
-  return true;
+  return px;
 }
 
-// Workspace slot of this thread: slots belong to the resident workgroup, not
-// to the tile, so the workspace is sized by the grid.
-__device__ __forceinline__ int slot_index() { return blockIdx.x * kSweepThreads + threadIdx.x; }
+// LDS of the windowed kernels.  The compiled windows have static arrays with
+// one row pitch for every tile shape, so window offsets are immediates; any
+// other window gets a launch-time block (window_lds_bytes) sized by its own
+// radius, so a small one leaves room for more workgroups.
+template <int R_, int S_>
+struct WinLds {
+  static constexpr int kTileWords = R_ >= 0 ? TileSize<R_>::kWords : 1;
+  static constexpr int kSpWords = R_ >= 0 ? SpSize<R_, S_>::kFloats : 1;
+  uint32_t tile[kTileWords];
+  float spl[kSpWords];
+  float ct[256];
+};
+extern __shared__ uint32_t win_dyn[];
+
+template <int R_, int S_>
+__device__ __forceinline__ uint32_t* lds_tile(WinLds<R_, S_>& l, VPtr v) {
+  if constexpr (R_ >= 0) return l.tile;
+  else return win_dyn + v->nwin * v->nwin;
+}
+template <int R_, int S_>
+__device__ __forceinline__ float* lds_spl(WinLds<R_, S_>& l) {
+  if constexpr (R_ >= 0) return l.spl;
+  else return (float*)win_dyn;
+}
+template <int R_>
+__device__ __forceinline__ int tile_pitch(int R, int lw) {
+  if constexpr (R_ >= 0) return TileSize<R_>::kPitch;
+  else return (1 << lw) + 2 * R;
+}
 
 // ---------------------------------------------------------------------------
 // init: random (best of init_samples) or given depth/normal, then InitConf
 
 template <int R_, int S_, int STORE, int RCP>
-__device__ __forceinline__ void init_tile(const Ctx& cx, uint32_t* tile, float* ct, float* spl) {
+__device__ __forceinline__ void init_tile(const Ctx& cx, WinLds<R_, S_>& lds) {
   const VPtr v = cx.v;
   const uint32_t pass = cx.pass;
   const int R = R_ >= 0 ? R_ : v->radius;
-  Pix px;
-  const int tw = R_ >= 0 ? TileSize<R_>::kPitch : (1 << kTileLog2WMax) + 2 * R;
-  if (!setup_pass(cx, R, tw, tile, ct, spl, px)) return;
+  uint32_t* tile = lds_tile<R_, S_>(lds, v);
+  float* spl = lds_spl<R_, S_>(lds);
+  float* ct = lds.ct;
+  const int tw = tile_pitch<R_>(R, cx.lw);
+  const Geo geo = stage_tile(cx, R, tw, tile, ct, spl);
+  __syncthreads();
+  const int slot = threadIdx.x;
+  int lrow, lcol;
+  geo.pixel(slot, lrow, lcol);
+  if (slot >= (1 << cx.lpx) || geo.row0 + lrow >= v->H || geo.col0 + lcol >= v->W) return;
+  const Pix px = make_pix(v, geo, tile, R, lrow, lcol,
+                          ld_f4(v->refm, (geo.row0 + lrow) * v->W + geo.col0 + lcol));
   const uint32_t* wt = tile + px.lrow * tw + px.lcol;
   const int N = v->N;
   const int plane = v->W * v->H;
-  Ws ws{cx.ws, cx.ws_slots, slot_index(), N};
+  Ws ws{cx.ws, 1 << cx.lpx, N};
   Counters cnt;
   pm_rng g;
   pm_rng_init(&g, v->seed, (uint32_t)v->view_id, (uint32_t)px.p, pass);
@@ -764,7 +818,7 @@ __device__ __forceinline__ void init_tile(const Ctx& cx, uint32_t* tile, float* 
       if (hn[0] * px.np0 + hn[1] * px.np1 + hn[2] * 1.0f >= 0.0f) random_normal(&g, px.np0, px.np1, hn);
     }
     for (int i = 0; i < N; ++i) {
-      ws.M(cx.color, i) = mv_cost<R_, S_, STORE, RCP>(v, i, px, wt, tw, ct, spl, hn[0], hn[1], hn[2], hd, v->refK, cnt);
+      ws.M(0, i, slot) = mv_cost<R_, S_, STORE, RCP>(v, i, px, wt, tw, ct, spl, hn[0], hn[1], hn[2], hd, v->refK, cnt);
     }
     // thk smallest costs in stable ascending order (= the reference's
     // bubble sort, kernel_functions.cu:1588-1597)
@@ -775,7 +829,7 @@ __device__ __forceinline__ void init_tile(const Ctx& cx, uint32_t* tile, float* 
       float bv = 0.0f;
       for (int i = 0; i < N; ++i) {
         if ((taken >> i) & 1u) continue;
-        const float cv = ws.M(cx.color, i);
+        const float cv = ws.M(0, i, slot);
         if (bi < 0 || cv < bv) {
           bi = i;
           bv = cv;
@@ -792,7 +846,7 @@ __device__ __forceinline__ void init_tile(const Ctx& cx, uint32_t* tile, float* 
       bn[0] = hn[0];
       bn[1] = hn[1];
       bn[2] = hn[2];
-      for (int i = 0; i < N; ++i) ws.RM(cx.color, i) = ws.M(cx.color, i);
+      for (int i = 0; i < N; ++i) ws.RM(0, i, slot) = ws.M(0, i, slot);
     }
   }
   G(v->depth)[px.p] = bd;
@@ -801,18 +855,195 @@ __device__ __forceinline__ void init_tile(const Ctx& cx, uint32_t* tile, float* 
   G(v->normal)[2 * plane + px.p] = bn[2];
   G(v->conf)[px.p] = best_conf;
   G(v->view_sel)[px.p] = best_sel;
-  for (int i = 0; i < N; ++i) G(v->cost)[i * plane + px.p] = ws.RM(cx.color, i);
+  for (int i = 0; i < N; ++i) G(v->cost)[i * plane + px.p] = ws.RM(0, i, slot);
   flush_counters(v, cnt);
 }
 
 template <int R_, int S_, int STORE, int RCP>
 __global__ __launch_bounds__(kSweepThreads) void k_init(const LaunchTable* __restrict__ lt) {
-  __shared__ uint32_t tile[TileSize<R_>::kWords];
-  __shared__ float ct[256];
-  __shared__ float spl[SpSize<R_, S_>::kFloats];
+  __shared__ WinLds<R_, S_> lds;
   __shared__ int next;
   for (int t = claim_tile(lt, &next); t >= 0; t = claim_tile(lt, &next))
-    init_tile<R_, S_, STORE, RCP>(resolve(lt, t), tile, ct, spl);
+    init_tile<R_, S_, STORE, RCP>(resolve(lt, t), lds);
+}
+
+// ---------------------------------------------------------------------------
+// evaluations shared by a workgroup
+//
+// What bounds the sweep is the VALU work of the window walks, so every walk
+// should serve 64 lanes that need it.  The pixels of a tile need different
+// evaluations (a candidate is missing, a source is not selected, a hypothesis
+// can no longer win), and a wave that keeps to its own 64 pixels walks the
+// union of what they need.  Here the (hypothesis, pixel) pairs that are needed
+// are listed in LDS, in order of pixel within a hypothesis so that 64
+// consecutive pairs still read neighbouring texels, and the four waves take
+// the list in units of one source x 64 pairs.  The source is uniform across a
+// unit: its pose and texture stay in scalar registers.  Listing also leaves
+// nothing of a pixel live across a walk but what the walk reads (122 VGPRs,
+// 4 waves per SIMD; one thread per pixel took 147 and 3).
+// Run of a 1920x1080 view (10 sources, 15x15, 8 iterations): one thread per
+// pixel 464 ms, here 342 ms.  160x120 (2 sources, 11x11 step 2, 5 iterations),
+// where the four waves share 64 pixels: 2.33 against 1.15 ms.
+
+// Per-workgroup LDS beside the window's: what the pairs need of a pixel.
+struct PassLds {
+  f4v refm[kSweepThreads];                    // {mu_r, var_r, 1/sum_w, err_r}
+  uint16_t list[kMaxHyp * kSweepThreads];     // pairs: hypothesis << 8 | pixel
+  float cost[kNumRefine * kSweepThreads];     // costs of a step, [source of the step][hypothesis][pixel]
+  uint32_t sel[kSweepThreads];                // selected sources
+  uint32_t bits[kSweepThreads];               // valid candidates
+  float bar[kSweepThreads];                   // cost a hypothesis has to reach
+  uint32_t win[kSweepThreads];                // workspace slot of the winner | its index << 8, or kNone
+  uint8_t own[4][kSweepThreads];              // per wave: pixels of a source
+  int count[2][4];                            // pairs per source of a step
+};
+constexpr uint32_t kNone = 0xffffffffu;
+constexpr int kLoTrials = 5;                    // trials of the local optimisation
+
+__device__ __forceinline__ int lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
+// Lanes below this one in the mask.
+__device__ __forceinline__ int rank_in(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+// LDS written by some lanes of a wave, read by others of the same wave.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Cost of hypothesis h of tile pixel q against source i.
+template <int R_, int S_, int STORE, int RCP>
+__device__ __forceinline__ float eval_pair(VPtr v, const Geo& geo, const PassLds& L, const uint32_t* tile,
+                                           const float* ct, const float* spl, int R, int q, f4v h, int i,
+                                           K4<float>* Kgeo, Counters& cnt) {
+  int lrow, lcol;
+  geo.pixel(q, lrow, lcol);
+  const Pix px = make_pix(v, geo, tile, R, lrow, lcol, L.refm[q]);
+  const int pitch = R_ >= 0 ? TileSize<R_>::kPitch : geo.pitch;
+  return mv_cost<R_, S_, STORE, RCP>(v, i, px, tile + lrow * pitch + lcol, pitch, ct, spl, h.x, h.y, h.z, h.w, Kgeo, cnt);
+}
+
+// Hypotheses against the sources their pixels selected, source by source in
+// ascending order, `group` sources a step.  Hypothesis k (0..nk-1) of a pixel
+// is workspace slot slot0 + k; the running sums are those of the plain loop.
+// A cost is >= 0 and a float sum of non-negative terms never decreases, so
+// once dead(sum) holds the hypothesis cannot win and its further evaluations
+// are left out (unless `all`: then every hypothesis meets every source).
+// Owner threads (pixel px, hypotheses part, part + parts, ...) keep the sums;
+// they return in sum[j] / alive bit j for hypothesis part + j * parts.
+// Costs go to store(k, i, px, cost) and, summed, through weight(i).
+template <int R_, int S_, int STORE, int RCP, int NK, typename Weight, typename Dead, typename Store>
+__device__ __forceinline__ uint32_t eval_selected(VPtr v, const Geo& geo, PassLds& L, const Ws& ws, const uint32_t* tile,
+                                                  const float* ct, const float* spl, int R, int px, int part, int parts,
+                                                  int slot0, uint32_t sel, bool all, int group, float (&sum)[NK],
+                                                  Weight weight, Dead dead, Store store, Counters& cnt) {
+  const int N = v->N, npx = ws.npx;
+  const int wave = wave_id(), lane = lane_id();
+  uint32_t alive = 0;
+#pragma unroll
+  for (int j = 0; j < NK; ++j) {
+    sum[j] = 0.0f;
+    if (part + j * parts < NK) alive |= 1u << j;
+  }
+  if (!all && sel == 0) alive = 0;
+  if (threadIdx.x < 8) (&L.count[0][0])[threadIdx.x] = 0;
+  __syncthreads();
+  const int cap = NK * npx;  // pairs of one source
+  for (int i0 = 0, step = 0; i0 < N; i0 += group, step ^= 1) {
+    for (int g = 0; g < group && i0 + g < N; ++g) {
+      const bool want = all || ((sel >> (i0 + g)) & 1u);
+      int total = 0;
+#pragma unroll
+      for (int j = 0; j < NK; ++j) total += __popcll(__ballot(want && ((alive >> j) & 1u)));
+      if (total == 0) continue;
+      int base = 0;
+      if (lane == 0) base = atomicAdd(&L.count[step][g], total);
+      base = g * cap + __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+      for (int j = 0; j < NK; ++j) {
+        const bool on = want && ((alive >> j) & 1u);
+        const uint64_t m = __ballot(on);
+        if (on) L.list[base + rank_in(m)] = (uint16_t)(((part + j * parts) << 8) | px);
+        base += __popcll(m);
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x < 4) L.count[step ^ 1][threadIdx.x] = 0;
+    int g = 0, n = __builtin_amdgcn_readfirstlane(L.count[step][0]), u0 = 0;
+    for (int u = wave;; u += 4) {
+      while (g < group && u >= u0 + ((n + 63) >> 6)) {
+        u0 += (n + 63) >> 6;
+        ++g;
+        n = g < group ? __builtin_amdgcn_readfirstlane(L.count[step][g]) : 0;
+      }
+      if (g >= group) break;
+      const int e = (u - u0) * 64 + lane;
+      if (e < n) {
+        const int code = L.list[g * cap + e];
+        const int k = code >> 8, q = code & 0xff;
+        const float m = eval_pair<R_, S_, STORE, RCP>(v, geo, L, tile, ct, spl, R, q, ws.hyp(slot0 + k, q), i0 + g,
+                                                      v->refK, cnt);
+        L.cost[(g * NK + k) * npx + q] = m;
+        store(k, i0 + g, q, m);
+      }
+    }
+    __syncthreads();
+    for (int g2 = 0; g2 < group && i0 + g2 < N; ++g2) {
+      const bool picked = (sel >> (i0 + g2)) & 1u;
+      if (!picked && !all) continue;
+      const float w = picked ? weight(i0 + g2) : 0.0f;
+#pragma unroll
+      for (int j = 0; j < NK; ++j) {
+        if (!((alive >> j) & 1u)) continue;
+        sum[j] = sum[j] + w * L.cost[(g2 * NK + part + j * parts) * npx + px];
+        if (!all && dead(sum[j])) alive &= ~(1u << j);
+      }
+    }
+  }
+  return alive;
+}
+
+// Costs of the winners against the sources their pixels did not select, into
+// the cost maps.  Each wave takes whole sources; no barrier inside.
+template <int R_, int S_, int STORE, int RCP>
+__device__ __forceinline__ void eval_unselected(VPtr v, const Geo& geo, PassLds& L, const Ws& ws, const uint32_t* tile,
+                                                const float* ct, const float* spl, int R, K4<float>* Kgeo,
+                                                Counters& cnt) {
+  const int N = v->N, W = v->W, plane = v->W * v->H;
+  const int wave = wave_id(), lane = lane_id();
+  uint8_t* own = L.own[wave];
+  for (int i = wave; i < N; i += 4) {
+    int n = 0;
+    for (int q0 = 0; q0 < ws.npx; q0 += 64) {
+      const int q = q0 + lane;
+      const bool on = L.win[q] != kNone && !((L.sel[q] >> i) & 1u);
+      const uint64_t m = __ballot(on);
+      if (on) own[n + rank_in(m)] = (uint8_t)q;
+      n += __popcll(m);
+    }
+    wave_lds_sync();
+    for (int e0 = 0; e0 < n; e0 += 64) {
+      if (e0 + lane < n) {
+        const int q = own[e0 + lane];
+        const float m = eval_pair<R_, S_, STORE, RCP>(v, geo, L, tile, ct, spl, R, q, ws.hyp((int)(L.win[q] & 0xffu), q),
+                                                      i, Kgeo, cnt);
+        int lrow, lcol;
+        geo.pixel(q, lrow, lcol);
+        G(v->cost)[i * plane + (geo.row0 + lrow) * W + geo.col0 + lcol] = m;
+      }
+    }
+    wave_lds_sync();
+  }
+}
+
+// Whether every cost is a finite number >= 0 (NCC is in [0, 2]; the geometric
+// term in [0, its maximum] times the regulariser): then a zero weight removes
+// a source from a weighted sum exactly, and partial sums never decrease.
+__device__ __forceinline__ bool costs_bounded(VPtr v) {
+  return !v->geom || (v->geom_regularizer >= 0.0f && v->geom_max_cost >= 0.0f &&
+                      v->geom_regularizer * v->geom_max_cost < 1e30f);
 }
 
 // ---------------------------------------------------------------------------
@@ -826,394 +1057,490 @@ __global__ __launch_bounds__(kSweepThreads) void k_init(const LaunchTable* __res
 #define PM_SWEEP_OCC
 #endif
 
+// Samples of the CDF held in registers at a time.
+constexpr int kDraws = 16;
+
 template <int R_, int S_, int STORE, int RCP>
-__device__ __forceinline__ void sweep_tile(const Ctx& cx, uint32_t* tile, float* ct, float* spl) {
+__device__ __forceinline__ void sweep_tile(const Ctx& cx, WinLds<R_, S_>& lds, PassLds& L) {
   const VPtr v = cx.v;
-  const uint32_t pass = cx.pass;
-  const float th_mc = cx.th_mc;
   const int R = R_ >= 0 ? R_ : v->radius;
-  Pix px;
-  const int tw = R_ >= 0 ? TileSize<R_>::kPitch : (1 << kTileLog2WMax) + 2 * R;
-  if (!setup_pass(cx, R, tw, tile, ct, spl, px)) return;
-  const uint32_t* wt = tile + px.lrow * tw + px.lcol;
+  uint32_t* tile = lds_tile<R_, S_>(lds, v);
+  float* spl = lds_spl<R_, S_>(lds);
+  const float* ct = lds.ct;
   const int W = v->W, H = v->H, N = v->N;
   const int plane = W * H;
-  const int p = px.p, row = px.row, col = px.col;
-  K4<float>* iK = v->refInvK;
-  Ws ws{cx.ws, cx.ws_slots, slot_index(), N};
+  const int npx = 1 << cx.lpx, parts = kSweepThreads >> cx.lpx;
+  const int px = threadIdx.x & (npx - 1), part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> cx.lpx));  // thread: a share of a pixel's bookkeeping
+  const int wave = wave_id(), lane = lane_id();
+  const Geo geo = stage_tile(cx, R, tile_pitch<R_>(R, cx.lw), tile, lds.ct, spl);
+  const Ws ws{cx.ws, npx, N};
   Counters cnt;
+  int lrow, lcol;
+  geo.pixel(px, lrow, lcol);
+  const int row = geo.row0 + lrow, col = geo.col0 + lcol;
+  const bool in = row < H && col < W;
+  const int p = row * W + col;
+  if (part == 0) {
+    if (in) L.refm[px] = ld_f4(v->refm, p);
+    L.bits[px] = in ? 1u : 0u;
+    L.sel[px] = 0u;
+    L.win[px] = kNone;
+  }
+  if (threadIdx.x == 0) L.count[0][0] = 0;
+  __syncthreads();
 
-  const float vd[3] = {px.np0, px.np1, 1.0f};
+  K4<float>* iK = v->refInvK;
+  const float vd[3] = {iK[0] * (float)col + iK[1], iK[2] * (float)row + iK[3], 1.0f};
   const float inv_view_len = 1.0f / sqrtf(vd[0] * vd[0] + vd[1] * vd[1] + vd[2] * vd[2]);
+  const bool full = v->counters != nullptr || !costs_bounded(v);  // counted runs make every evaluation
 
-  // candidates
-  int nh = 0;
-  ws.hyp(0, 0) = G(v->normal)[p];
-  ws.hyp(0, 1) = G(v->normal)[plane + p];
-  ws.hyp(0, 2) = G(v->normal)[2 * plane + p];
-  ws.hyp(0, 3) = G(v->depth)[p];
-  nh = 1;
-  if (G(v->grad_ok)[p]) {
-    float nconf[4];
-    int order[4];
-    int nvalid = 0;
+  // candidates: slot 0 the current hypothesis, 1 and 2 the better of the
+  // 4-neighbours, 3 + g the best of direction g
+  if (in) {
+    uint32_t valid = 0;
+    for (int task = part; task < 9; task += parts) {
+      if (task == 0) {
+        ws.hyp(0, px) = f4v{G(v->normal)[p], G(v->normal)[plane + p], G(v->normal)[2 * plane + p], G(v->depth)[p]};
+        if (!G(v->grad_ok)[p]) continue;
+        float nconf[4];
+        int order[4];
+        int nvalid = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      order[k] = k;
-      const int u = col + c_neighbor_offs[k][1], w = row + c_neighbor_offs[k][0];
-      if (u < 0 || u >= W || w < 0 || w >= H) {
-        nconf[k] = PM_FLT_MAX;
-        continue;
-      }
-      nvalid++;
-      nconf[k] = G(v->conf)[w * W + u];
-    }
+        for (int k = 0; k < 4; ++k) {
+          order[k] = k;
+          const int u = col + c_neighbor_offs[k][1], w = row + c_neighbor_offs[k][0];
+          if (u < 0 || u >= W || w < 0 || w >= H) {
+            nconf[k] = PM_FLT_MAX;
+            continue;
+          }
+          nvalid++;
+          nconf[k] = G(v->conf)[w * W + u];
+        }
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
+        for (int a = 0; a < 3; ++a) {
 #pragma unroll
-      for (int b = 0; b < 3 - a; ++b) {
-        if (nconf[b] > nconf[b + 1]) {
-          const float t = nconf[b];
-          nconf[b] = nconf[b + 1];
-          nconf[b + 1] = t;
-          const int o = order[b];
-          order[b] = order[b + 1];
-          order[b + 1] = o;
+          for (int b = 0; b < 3 - a; ++b) {
+            if (nconf[b] > nconf[b + 1]) {
+              const float t = nconf[b];
+              nconf[b] = nconf[b + 1];
+              nconf[b + 1] = t;
+              const int o = order[b];
+              order[b] = order[b + 1];
+              order[b + 1] = o;
+            }
+          }
+        }
+        if (nvalid > 2) nvalid = 2;
+        for (int k = 0; k < nvalid; ++k) {
+          const int idx = k == 0 ? order[0] : order[1];
+          const int u = col + c_neighbor_offs[idx][1], w = row + c_neighbor_offs[idx][0];
+          const int q = w * W + u;
+          float nn[3] = {G(v->normal)[q], G(v->normal)[plane + q], G(v->normal)[2 * plane + q]};
+          correct_normal(nn, vd, inv_view_len);
+          const float dd = propagate_depth(G(v->depth)[q], nn, iK, w, u, vd[0], vd[1]);
+          ws.hyp(1 + k, px) = f4v{nn[0], nn[1], nn[2], dd};
+          valid |= 2u << k;
+        }
+      } else {
+        const int gi = task - 1;
+        float best_conf = PM_FLT_MAX;
+        int br = 0, bc = 0;
+#pragma unroll
+        for (int f = 0; f < 10; ++f) {
+          const int nr = row + c_dir_samples[gi][2 * f];
+          const int ncn = col + c_dir_samples[gi][2 * f + 1];
+          if (nr < 0 || nr >= H || ncn < 0 || ncn >= W) continue;
+          const float cv = G(v->conf)[nr * W + ncn];
+          if (best_conf > cv) {
+            best_conf = cv;
+            br = nr;
+            bc = ncn;
+          }
+        }
+        if (best_conf < PM_FLT_MAX) {
+          const int q = br * W + bc;
+          float nn[3] = {G(v->normal)[q], G(v->normal)[plane + q], G(v->normal)[2 * plane + q]};
+          correct_normal(nn, vd, inv_view_len);
+          const float dd = propagate_depth(G(v->depth)[q], nn, iK, br, bc, vd[0], vd[1]);
+          ws.hyp(3 + gi, px) = f4v{nn[0], nn[1], nn[2], dd};
+          valid |= 8u << gi;
         }
       }
     }
-    if (nvalid > 2) nvalid = 2;
-    for (int k = 0; k < nvalid; ++k) {
-      const int idx = order[k];
-      const int u = col + c_neighbor_offs[idx][1], w = row + c_neighbor_offs[idx][0];
-      const int q = w * W + u;
-      float nn[3] = {G(v->normal)[q], G(v->normal)[plane + q], G(v->normal)[2 * plane + q]};
-      correct_normal(nn, vd, inv_view_len);
-      const float dd = propagate_depth(G(v->depth)[q], nn, iK, w, u, px.np0, px.np1);
-      ws.hyp(nh, 0) = nn[0];
-      ws.hyp(nh, 1) = nn[1];
-      ws.hyp(nh, 2) = nn[2];
-      ws.hyp(nh, 3) = dd;
-      nh++;
-    }
+    if (valid) atomicOr(&L.bits[px], valid);
   }
-  for (int gi = 0; gi < 8; ++gi) {
-    float best_conf = PM_FLT_MAX;
-    int br = 0, bc = 0;
-#pragma unroll
-    for (int f = 0; f < 10; ++f) {
-      const int nr = row + c_dir_samples[gi][2 * f];
-      const int ncn = col + c_dir_samples[gi][2 * f + 1];
-      if (nr < 0 || nr >= H || ncn < 0 || ncn >= W) continue;
-      const float cv = G(v->conf)[nr * W + ncn];
-      if (best_conf > cv) {
-        best_conf = cv;
-        br = nr;
-        bc = ncn;
-      }
-    }
-    if (best_conf < PM_FLT_MAX) {
-      const int q = br * W + bc;
-      float nn[3] = {G(v->normal)[q], G(v->normal)[plane + q], G(v->normal)[2 * plane + q]};
-      correct_normal(nn, vd, inv_view_len);
-      const float dd = propagate_depth(G(v->depth)[q], nn, iK, br, bc, px.np0, px.np1);
-      ws.hyp(nh, 0) = nn[0];
-      ws.hyp(nh, 1) = nn[1];
-      ws.hyp(nh, 2) = nn[2];
-      ws.hyp(nh, 3) = dd;
-      nh++;
-    }
-  }
+  __syncthreads();
 
-  // cost matrix, source-major so consecutive evaluations share a source
-  for (int i = 0; i < N; ++i) {
-    ws.M(0, i) = G(v->cost)[i * plane + p];
+  // the candidates' pairs; then the cost matrix, source by source
+  if (wave * 64 < npx) {
+    const uint32_t b = L.bits[wave * 64 + lane];
+    int total = 0;
+    for (int k = 1; k < kMaxHyp; ++k) total += __popcll(__ballot((b >> k) & 1u));
+    int base = 0;
+    if (lane == 0) base = atomicAdd(&L.count[0][0], total);
+    base = __builtin_amdgcn_readfirstlane(base);
     for (int k = 1; k < kMaxHyp; ++k) {
-      if (k < nh) {
-        ws.M(k, i) = mv_cost<R_, S_, STORE, RCP>(v, i, px, wt, tw, ct, spl, ws.hyp(k, 0), ws.hyp(k, 1), ws.hyp(k, 2),
-                                                 ws.hyp(k, 3), v->refK, cnt);
-      }
+      const uint64_t m = __ballot((b >> k) & 1u);
+      if ((b >> k) & 1u) L.list[base + rank_in(m)] = (uint16_t)((k << 8) | (wave * 64 + lane));
+      base += __popcll(m);
     }
   }
+  __syncthreads();
+  {
+    const int n = __builtin_amdgcn_readfirstlane(L.count[0][0]);
+    const int chunks = (n + 63) >> 6;
+    int i = 0, c = wave;
+    for (;;) {
+      while (c >= chunks && i < N) {
+        c -= chunks;
+        ++i;
+        if (chunks == 0) i = N;
+      }
+      if (i >= N) break;
+      const int e = c * 64 + lane;
+      if (e < n) {
+        const int code = L.list[e];
+        const int k = code >> 8, q = code & 0xff;
+        ws.M(k, i, q) = eval_pair<R_, S_, STORE, RCP>(v, geo, L, tile, ct, spl, R, q, ws.hyp(k, q), i, v->refK, cnt);
+      }
+      c += 4;
+    }
+  }
+  __syncthreads();
 
   // view selection (kernel_functions.cu:2364-2426)
-  uint32_t flags = 0;
-  for (int i = 0; i < N; ++i) {
-    float pr = 0.0f;
-    int n1 = 0, n2 = 0;
-    for (int k = 0; k < nh; ++k) {
-      const float cv = ws.M(k, i);
-      pr = pr + pm_expf(-(cv * cv) * v->inv_beta2);
-      n1 += (cv < th_mc);
-      n2 += (cv > v->max_ncc_matching_cost);
+  const uint32_t valid = L.bits[px];  // 0 outside the image
+  if (in) {
+    uint32_t flags = 0;
+    for (int i = part; i < N; i += parts) {
+      const float c0 = G(v->cost)[i * plane + p];
+      ws.M(0, i, px) = c0;
+      float pr = 0.0f;
+      int n1 = 0, n2 = 0;
+#pragma unroll
+      for (int k = 0; k < kMaxHyp; ++k) {
+        if (!((valid >> k) & 1u)) continue;
+        const float cv = k == 0 ? c0 : ws.M(k, i, px);
+        pr = pr + pm_expf(-(cv * cv) * v->inv_beta2);
+        n1 += (cv < cx.th_mc);
+        n2 += (cv > v->max_ncc_matching_cost);
+      }
+      ws.Wt(i, px) = pr;
+      if (n1 >= v->num_good && n2 <= v->num_bad) flags |= 1u << i;
     }
-    ws.Wt(i) = pr;
-    if (n1 >= v->num_good && n2 <= v->num_bad) flags |= 1u << i;
+    if (flags) atomicOr(&L.sel[px], flags);
   }
-  if (flags == 0) {
-    flush_counters(v, cnt, true);
-    return;
-  }
-  float psum = 0.0f;
-  for (int i = 0; i < N; ++i) {
-    const float pr = ((flags >> i) & 1u) ? ws.Wt(i) : 0.0f;
-    psum = psum + pr;
-  }
-  const float inv_psum = 1.0f / psum;
-  float cum = 0.0f;
-  for (int i = 0; i < N; ++i) {
-    const float pr = ((flags >> i) & 1u) ? ws.Wt(i) : 0.0f;
-    cum = cum + pr * inv_psum;
-    ws.Wt(i) = cum;
-    ws.RM(0, i) = 0.0f;
-  }
+  __syncthreads();
+
+  // the draws: a pixel's first thread picks the sources (L.sel: flags in,
+  // selected sources out) and keeps the stream for the refinement
+  const bool once = v->random_optimization != 0;  // a picked source weighs 1, or its number of picks
+  uint32_t sel = L.sel[px];
   pm_rng g;
-  pm_rng_init(&g, v->seed, (uint32_t)v->view_id, (uint32_t)p, pass);
-  for (int smp = 0; smp < v->num_samples; ++smp) {
-    const float rp = pm_rng_uniform(&g) - PM_FLT_EPSILON;
-    for (int i = 0; i < N; ++i) {
-      if (ws.Wt(i) > rp) {
-        ws.RM(0, i) = v->random_optimization ? 1.0f : ws.RM(0, i) + 1.0f;
-        break;
+  float norm = 0.0f;  // 1 / sum of the weights
+  if (part == 0 && sel != 0) {
+    const uint32_t flags = sel;
+    float psum = 0.0f;
+    for (int i = 0; i < N; ++i) psum = psum + (((flags >> i) & 1u) ? ws.Wt(i, px) : 0.0f);
+    const float inv_psum = 1.0f / psum;
+    pm_rng_init(&g, v->seed, (uint32_t)v->view_id, (uint32_t)p, cx.pass);
+    uint32_t picked = 0;
+    int picks = 0;
+    for (int s0 = 0; s0 < v->num_samples; s0 += kDraws) {
+      float rp[kDraws];
+      const int ns = v->num_samples - s0;
+#pragma unroll
+      for (int s = 0; s < kDraws; ++s) {
+        rp[s] = INFINITY;
+        if (s < ns) rp[s] = pm_rng_uniform(&g) - PM_FLT_EPSILON;
+      }
+      // each draw picks the first source whose CDF exceeds it
+      float cum = 0.0f;
+      for (int i = 0; i < N; ++i) {
+        const float pr = ((flags >> i) & 1u) ? ws.Wt(i, px) : 0.0f;
+        cum = cum + pr * inv_psum;
+        int hits = 0;
+#pragma unroll
+        for (int s = 0; s < kDraws; ++s) {
+          if (cum > rp[s]) {
+            hits++;
+            rp[s] = INFINITY;
+          }
+        }
+        if (!once) ws.RM(0, i, px) = (s0 > 0 ? ws.RM(0, i, px) : 0.0f) + (float)hits;
+        if (hits) picked |= 1u << i;
+        picks += hits;
+      }
+    }
+    const float wnorm = once ? (float)__popc(picked) : (float)picks;
+    if (wnorm <= 1e-5f) picked = 0;
+    else norm = 1.0f / wnorm;
+    if (!once && picked) {
+      for (int i = 0; i < N; ++i) ws.Wt(i, px) = ws.RM(0, i, px) * norm;
+    }
+    L.sel[px] = picked;
+    L.bar[px] = norm;
+  }
+  __syncthreads();
+  sel = L.sel[px];
+  norm = L.bar[px];
+  // weight of selected source i
+  auto weight = [&](int i) __attribute__((always_inline)) { return once ? norm : ws.Wt(i, px); };
+  int best = -1;
+  float minc = PM_FLT_MAX;
+  if (sel != 0) {
+    for (int k = part; k < kMaxHyp; k += parts) {
+      if (!((valid >> k) & 1u)) continue;
+      float cc = 0.0f;
+      for (int i = 0; i < N; ++i) {
+        if (full || ((sel >> i) & 1u)) cc = cc + (((sel >> i) & 1u) ? weight(i) : 0.0f) * ws.M(k, i, px);
+      }
+      if (cc <= minc) {
+        minc = cc;
+        best = k;
       }
     }
   }
-  float wnorm = 0.0f;
-  for (int i = 0; i < N; ++i) wnorm = wnorm + ws.RM(0, i);
-  if (wnorm <= 1e-5f) {
-    flush_counters(v, cnt, true);
-    return;
-  }
-  const float inv_wnorm = 1.0f / wnorm;
-  uint32_t sel = 0;
-  for (int i = 0; i < N; ++i) {
-    const float wv = ws.RM(0, i) * inv_wnorm;
-    ws.Wt(i) = wv;
-    if (wv > 0.0f) sel |= 1u << i;
-  }
-  int best = -1;
-  float minc = PM_FLT_MAX;
-  for (int k = 0; k < nh; ++k) {
-    float cc = 0.0f;
-    for (int i = 0; i < N; ++i) cc = cc + ws.Wt(i) * ws.M(k, i);
-    if (cc <= minc) {
-      minc = cc;
-      best = k;
+  if (parts > 1) {  // the last minimum wins: among equals the largest k
+    float* pc = L.cost;
+    int* pk = (int*)(L.cost + kSweepThreads);
+    pc[threadIdx.x] = minc;
+    pk[threadIdx.x] = best;
+    __syncthreads();
+    for (int o = 0; o < parts; ++o) {
+      const float c2 = pc[o * npx + px];
+      const int k2 = pk[o * npx + px];
+      if (k2 >= 0 && (best < 0 || c2 < minc || (c2 == minc && k2 > best))) {
+        minc = c2;
+        best = k2;
+      }
     }
   }
-  G(v->view_sel)[p] = sel;
-  if (best < 0) best = 0;
-  float depth = ws.hyp(best, 3);
-  float normal[3] = {ws.hyp(best, 0), ws.hyp(best, 1), ws.hyp(best, 2)};
-
-  // refinement hypotheses (kernel_functions.cu:2449-2486)
-  const float dlo = (1.0f - v->random_depth_ratio) * depth;
-  const float dhi = (1.0f + v->random_depth_ratio) * depth;
-  const float nd = random_depth(&g, dlo, dhi);
-  float nn[3];
-  perturb_normal(&g, normal, v->angle1, v->angle2, nn);
-  correct_normal(nn, vd, inv_view_len);
-  const float rd = random_depth(&g, v->depth_min, v->depth_max_eff);
-  float rn[3];
-  random_normal(&g, vd[0], vd[1], rn);
-  correct_normal(rn, vd, inv_view_len);
-  const int hb = kMaxHyp;  // refinement hypotheses stored after the candidates
-  ws.hyp(hb + 0, 0) = normal[0];
-  ws.hyp(hb + 0, 1) = normal[1];
-  ws.hyp(hb + 0, 2) = normal[2];
-  ws.hyp(hb + 0, 3) = depth;
-  ws.hyp(hb + 1, 0) = nn[0];
-  ws.hyp(hb + 1, 1) = nn[1];
-  ws.hyp(hb + 1, 2) = nn[2];
-  ws.hyp(hb + 1, 3) = depth;
-  ws.hyp(hb + 2, 0) = normal[0];
-  ws.hyp(hb + 2, 1) = normal[1];
-  ws.hyp(hb + 2, 2) = normal[2];
-  ws.hyp(hb + 2, 3) = nd;
-  ws.hyp(hb + 3, 0) = rn[0];
-  ws.hyp(hb + 3, 1) = rn[1];
-  ws.hyp(hb + 3, 2) = rn[2];
-  ws.hyp(hb + 3, 3) = depth;
-  ws.hyp(hb + 4, 0) = normal[0];
-  ws.hyp(hb + 4, 1) = normal[1];
-  ws.hyp(hb + 4, 2) = normal[2];
-  ws.hyp(hb + 4, 3) = rd;
-
-  float rc0 = 0.0f;
-  for (int i = 0; i < N; ++i) {
-    const float m = ws.M(best, i);
-    ws.RM(0, i) = m;
-    rc0 = rc0 + ws.Wt(i) * m;
+  float rc0 = minc;
+  if (sel != 0 && best < 0) {  // no sum below FLT_MAX
+    best = 0;
+    rc0 = 0.0f;
+    for (int i = 0; i < N; ++i) rc0 = rc0 + (((sel >> i) & 1u) ? weight(i) : 0.0f) * ws.M(0, i, px);
   }
-  for (int i = 0; i < N; ++i) {
-    for (int k = 1; k < kNumRefine; ++k) {
-      ws.RM(k, i) = mv_cost<R_, S_, STORE, RCP>(v, i, px, wt, tw, ct, spl, ws.hyp(hb + k, 0), ws.hyp(hb + k, 1),
-                                                ws.hyp(hb + k, 2), ws.hyp(hb + k, 3), v->refK, cnt);
-    }
+
+  // refinement hypotheses (kernel_functions.cu:2449-2486): slots kMaxHyp + 1..4
+  const int hb = kMaxHyp;
+  if (part == 0 && sel != 0) {
+    G(v->view_sel)[p] = sel;
+    const f4v h = ws.hyp(best, px);
+    const float depth = h.w;
+    const float normal[3] = {h.x, h.y, h.z};
+    const float dlo = (1.0f - v->random_depth_ratio) * depth;
+    const float dhi = (1.0f + v->random_depth_ratio) * depth;
+    const float nd = random_depth(&g, dlo, dhi);
+    float nn[3];
+    perturb_normal(&g, normal, v->angle1, v->angle2, nn);
+    correct_normal(nn, vd, inv_view_len);
+    const float rd = random_depth(&g, v->depth_min, v->depth_max_eff);
+    float rn[3];
+    random_normal(&g, vd[0], vd[1], rn);
+    correct_normal(rn, vd, inv_view_len);
+    ws.hyp(hb + 1, px) = f4v{nn[0], nn[1], nn[2], depth};
+    ws.hyp(hb + 2, px) = f4v{normal[0], normal[1], normal[2], nd};
+    ws.hyp(hb + 3, px) = f4v{rn[0], rn[1], rn[2], depth};
+    ws.hyp(hb + 4, px) = f4v{normal[0], normal[1], normal[2], rd};
   }
+
+  // A refined hypothesis replaces the best candidate if its weighted sum is
+  // not above rc0; only the selected sources enter that sum.
+  float sum[kNumRefine - 1];
+  const uint32_t alive = eval_selected<R_, S_, STORE, RCP, kNumRefine - 1>(
+      v, geo, L, ws, tile, ct, spl, R, px, part, parts, hb + 1, sel, full && sel != 0, full ? 1 : parts, sum, weight,
+      [&](float s) __attribute__((always_inline)) { return s > rc0; },
+      [&](int k, int i, int q, float m) __attribute__((always_inline)) { ws.RM(k + 1, i, q) = m; }, cnt);
   int b2 = -1;
   minc = PM_FLT_MAX;
-  for (int k = 0; k < kNumRefine; ++k) {
-    float cc = rc0;
-    if (k > 0) {
-      cc = 0.0f;
-      for (int i = 0; i < N; ++i) cc = cc + ws.Wt(i) * ws.RM(k, i);
-    }
-    if (cc <= minc) {
-      minc = cc;
-      b2 = k;
+  if (rc0 <= minc) {
+    minc = rc0;
+    b2 = 0;
+  }
+#pragma unroll
+  for (int j = 0; j < kNumRefine - 1; ++j) {
+    if (((alive >> j) & 1u) && sum[j] <= minc) {
+      minc = sum[j];
+      b2 = part + j * parts + 1;
     }
   }
-  if (b2 < 0) {  // every refined cost NaN: the reference writes nothing
-    flush_counters(v, cnt, true);
-    return;
+  if (parts > 1) {
+    float* pc = L.cost;
+    int* pk = (int*)(L.cost + kSweepThreads);
+    __syncthreads();  // the sums are no longer read
+    pc[threadIdx.x] = minc;
+    pk[threadIdx.x] = b2;
+    __syncthreads();
+    for (int o = 0; o < parts; ++o) {
+      const float c2 = pc[o * npx + px];
+      const int k2 = pk[o * npx + px];
+      if (k2 >= 0 && (b2 < 0 || c2 < minc || (c2 == minc && k2 > b2))) {
+        minc = c2;
+        b2 = k2;
+      }
+    }
   }
-  G(v->conf)[p] = minc;
-  G(v->depth)[p] = ws.hyp(hb + b2, 3);
-  G(v->normal)[p] = ws.hyp(hb + b2, 0);
-  G(v->normal)[plane + p] = ws.hyp(hb + b2, 1);
-  G(v->normal)[2 * plane + p] = ws.hyp(hb + b2, 2);
-  for (int i = 0; i < N; ++i) G(v->cost)[i * plane + p] = ws.RM(b2, i);
+  if (sel == 0) b2 = -1;  // b2 < 0 otherwise: every cost NaN, the pixel keeps its state
+  if (part == 0) L.win[px] = b2 > 0 && !full ? (uint32_t)(hb + b2) : kNone;
+  __syncthreads();
+  if (b2 >= 0) {
+    if (part == 0) {
+      const f4v h = ws.hyp(b2 == 0 ? best : hb + b2, px);
+      G(v->conf)[p] = minc;
+      G(v->depth)[p] = h.w;
+      G(v->normal)[p] = h.x;
+      G(v->normal)[plane + p] = h.y;
+      G(v->normal)[2 * plane + p] = h.z;
+    }
+    for (int i = part; i < N; i += parts) {
+      if (b2 == 0) G(v->cost)[i * plane + p] = ws.M(best, i, px);
+      else if (full || ((sel >> i) & 1u)) G(v->cost)[i * plane + p] = ws.RM(b2, i, px);
+    }
+  }
+  eval_unselected<R_, S_, STORE, RCP>(v, geo, L, ws, tile, ct, spl, R, v->refK, cnt);
   flush_counters(v, cnt, true);
 }
 
 template <int R_, int S_, int STORE, int RCP>
 __global__ __launch_bounds__(kSweepThreads) PM_SWEEP_OCC void k_sweep(const LaunchTable* __restrict__ lt) {
-  __shared__ uint32_t tile[TileSize<R_>::kWords];
-  __shared__ float ct[256];
-  __shared__ float spl[SpSize<R_, S_>::kFloats];
+  __shared__ WinLds<R_, S_> lds;
+  __shared__ PassLds pass;
   __shared__ int next;
   for (int t = claim_tile(lt, &next); t >= 0; t = claim_tile(lt, &next))
-    sweep_tile<R_, S_, STORE, RCP>(resolve(lt, t), tile, ct, spl);
+    sweep_tile<R_, S_, STORE, RCP>(resolve(lt, t), lds, pass);
 }
 
 // ---------------------------------------------------------------------------
 // local optimisation
 
 template <int R_, int S_, int STORE, int RCP>
-__device__ __forceinline__ void local_opt_tile(const Ctx& cx, uint32_t* tile, float* ct, float* spl) {
+__device__ __forceinline__ void local_opt_tile(const Ctx& cx, WinLds<R_, S_>& lds, PassLds& L) {
   const VPtr v = cx.v;
-  const uint32_t pass = cx.pass;
   const int R = R_ >= 0 ? R_ : v->radius;
-  Pix px;
-  const int tw = R_ >= 0 ? TileSize<R_>::kPitch : (1 << kTileLog2WMax) + 2 * R;
-  if (!setup_pass(cx, R, tw, tile, ct, spl, px)) return;
-  const uint32_t* wt = tile + px.lrow * tw + px.lcol;
+  uint32_t* tile = lds_tile<R_, S_>(lds, v);
+  float* spl = lds_spl<R_, S_>(lds);
+  const float* ct = lds.ct;
   const int W = v->W, H = v->H, N = v->N;
   const int plane = W * H;
-  const int p = px.p, row = px.row, col = px.col;
-  Ws ws{cx.ws, cx.ws_slots, slot_index(), N};
+  const int npx = 1 << cx.lpx, parts = kSweepThreads >> cx.lpx;
+  const int px = threadIdx.x & (npx - 1), part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> cx.lpx));
+  const Geo geo = stage_tile(cx, R, tile_pitch<R_>(R, cx.lw), tile, lds.ct, spl);
+  const Ws ws{cx.ws, npx, N};
   Counters cnt;
-
-  float conf = G(v->conf)[p];
-  const float depth = G(v->depth)[p];
-  const float normal[3] = {G(v->normal)[p], G(v->normal)[plane + p], G(v->normal)[2 * plane + p]};
-  const uint32_t sel = G(v->view_sel)[p];
-  const float angle1 = (float)(4.0 * 0.0174532925199432);
-  const float angle2 = (float)(2.0 * 0.0174532925199432);
-  float low = depth, up = depth;
-  float m0 = normal[0], m1 = normal[1], m2 = normal[2];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int u = col + c_neighbor_offs[k][1], w = row + c_neighbor_offs[k][0];
-    if (u < 0 || u >= W || w < 0 || w >= H) continue;
-    const int q = w * W + u;
-    const float ndp = G(v->depth)[q];
-    m0 = m0 + G(v->normal)[q];
-    m1 = m1 + G(v->normal)[plane + q];
-    m2 = m2 + G(v->normal)[2 * plane + q];
-    if (ndp <= low) low = ndp;
-    if (ndp > up) up = ndp;
+  int lrow, lcol;
+  geo.pixel(px, lrow, lcol);
+  const int row = geo.row0 + lrow, col = geo.col0 + lcol;
+  const bool in = row < H && col < W;
+  const int p = row * W + col;
+  const uint32_t sel = in ? G(v->view_sel)[p] : 0u;
+  const float conf0 = in ? G(v->conf)[p] : 0.0f;
+  if (part == 0) {
+    if (in) L.refm[px] = ld_f4(v->refm, p);
+    L.sel[px] = sel;
+    L.win[px] = kNone;
   }
-  float mn[3] = {m0, m1, m2};
-  const float inv_norm = 1.0f / sqrtf(mn[0] * mn[0] + mn[1] * mn[1] + mn[2] * mn[2]);
-  mn[0] = mn[0] * inv_norm;
-  mn[1] = mn[1] * inv_norm;
-  mn[2] = mn[2] * inv_norm;
-  if (sel == 0) return;
-  pm_rng g;
-  pm_rng_init(&g, v->seed, (uint32_t)v->view_id, (uint32_t)p, pass);
-  for (int t = 0; t < 5; ++t) {
-    float hn[3];
-    const float hd = random_depth(&g, low, up);
-    perturb_normal(&g, mn, angle1, angle2, hn);
-    ws.hyp(t, 0) = hn[0];
-    ws.hyp(t, 1) = hn[1];
-    ws.hyp(t, 2) = hn[2];
-    ws.hyp(t, 3) = hd;
+  if (part == 0 && sel != 0) {
+    const float depth = G(v->depth)[p];
+    const float angle1 = (float)(4.0 * 0.0174532925199432);
+    const float angle2 = (float)(2.0 * 0.0174532925199432);
+    float low = depth, up = depth;
+    float m0 = G(v->normal)[p], m1 = G(v->normal)[plane + p], m2 = G(v->normal)[2 * plane + p];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int u = col + c_neighbor_offs[k][1], w = row + c_neighbor_offs[k][0];
+      if (u < 0 || u >= W || w < 0 || w >= H) continue;
+      const int q = w * W + u;
+      const float ndp = G(v->depth)[q];
+      m0 = m0 + G(v->normal)[q];
+      m1 = m1 + G(v->normal)[plane + q];
+      m2 = m2 + G(v->normal)[2 * plane + q];
+      if (ndp <= low) low = ndp;
+      if (ndp > up) up = ndp;
+    }
+    float mn[3] = {m0, m1, m2};
+    const float inv_norm = 1.0f / sqrtf(mn[0] * mn[0] + mn[1] * mn[1] + mn[2] * mn[2]);
+    mn[0] = mn[0] * inv_norm;
+    mn[1] = mn[1] * inv_norm;
+    mn[2] = mn[2] * inv_norm;
+    pm_rng g;
+    pm_rng_init(&g, v->seed, (uint32_t)v->view_id, (uint32_t)p, cx.pass);
+    for (int t = 0; t < kLoTrials; ++t) {
+      float hn[3];
+      const float hd = random_depth(&g, low, up);
+      perturb_normal(&g, mn, angle1, angle2, hn);
+      ws.hyp(t, px) = f4v{hn[0], hn[1], hn[2], hd};
+    }
   }
   // A trial's mean over the selected sources is its running sum / mw.
   // Costs are >= 0 (NCC in [0, 2], the geometric term scaled by a
   // non-negative regulariser) and a float sum of non-negative terms never
   // decreases, so once sum / mw >= the pixel's conf the trial cannot be
-  // taken: its remaining evaluations are skipped (a wave skips a walk when
-  // every lane has ruled the trial out).  The maps are those of the full
-  // evaluation; the transcription prunes the same evaluations.
+  // taken: its remaining evaluations are skipped.  The maps are those of the
+  // full evaluation; the transcription prunes the same evaluations (and a
+  // counted run takes one source a step, as it does).
   const float mw = (float)__popc(sel);
-  const float conf0 = conf;
   const bool prune = !v->geom || v->geom_regularizer >= 0.0f;
-  float part0 = 0.0f, part1 = 0.0f, part2 = 0.0f, part3 = 0.0f, part4 = 0.0f;
-  uint32_t live = 0x1fu;
-  for (int i = 0; i < N; ++i) {
-    if (!((sel >> i) & 1u)) continue;
-#pragma unroll 1
-    for (int t = 0; t < 5; ++t) {
-      if (!((live >> t) & 1u)) continue;
-      const float m = mv_cost<R_, S_, STORE, RCP>(v, i, px, wt, tw, ct, spl, ws.hyp(t, 0), ws.hyp(t, 1),
-                                                  ws.hyp(t, 2), ws.hyp(t, 3), v->refK, cnt);
-      ws.M(t, i) = m;
-      float sum;
-      if (t == 0) sum = part0 = part0 + m;
-      else if (t == 1) sum = part1 = part1 + m;
-      else if (t == 2) sum = part2 = part2 + m;
-      else if (t == 3) sum = part3 = part3 + m;
-      else sum = part4 = part4 + m;
-      if (prune && sum / mw >= conf0) live &= ~(1u << t);
-    }
-  }
+  float sum[kLoTrials];
+  const uint32_t alive = eval_selected<R_, S_, STORE, RCP, kLoTrials>(
+      v, geo, L, ws, tile, ct, spl, R, px, part, parts, 0, sel, false, v->counters != nullptr ? 1 : parts, sum,
+      [](int) __attribute__((always_inline)) { return 1.0f; },
+      [&](float s) __attribute__((always_inline)) { return prune && s / mw >= conf0; },
+      [&](int k, int i, int q, float m) __attribute__((always_inline)) { ws.M(k, i, q) = m; }, cnt);
+  // the first of the smallest means below the pixel's conf
+  float conf = conf0;
   int best = -1;
-  const float parts[5] = {part0, part1, part2, part3, part4};
 #pragma unroll
-  for (int t = 0; t < 5; ++t) {
-    if (!((live >> t) & 1u)) continue;
-    const float mconf = parts[t] / mw;
+  for (int j = 0; j < kLoTrials; ++j) {
+    if (!((alive >> j) & 1u)) continue;
+    const float mconf = sum[j] / mw;
     if (mconf < conf) {
       conf = mconf;
-      best = t;
+      best = part + j * parts;
     }
   }
-  if (best < 0) {
-    flush_counters(v, cnt);
-    return;
-  }
-  const float bd = ws.hyp(best, 3);
-  const float bn[3] = {ws.hyp(best, 0), ws.hyp(best, 1), ws.hyp(best, 2)};
-  G(v->conf)[p] = conf;
-  G(v->depth)[p] = bd;
-  G(v->normal)[p] = bn[0];
-  G(v->normal)[plane + p] = bn[1];
-  G(v->normal)[2 * plane + p] = bn[2];
-  K4<float>* Kgeo = v->compat_lo_geo_bug ? v->refInvK : v->refK;
-  for (int i = 0; i < N; ++i) {
-    float cv;
-    if ((sel >> i) & 1u) {
-      cv = ws.M(best, i);
-    } else {
-      cv = mv_cost<R_, S_, STORE, RCP>(v, i, px, wt, tw, ct, spl, bn[0], bn[1], bn[2], bd, Kgeo, cnt);
+  if (parts > 1) {
+    float* pc = L.cost;
+    int* pk = (int*)(L.cost + kSweepThreads);
+    __syncthreads();  // the sums are no longer read
+    pc[threadIdx.x] = conf;
+    pk[threadIdx.x] = best;
+    __syncthreads();
+    for (int o = 0; o < parts; ++o) {
+      const float c2 = pc[o * npx + px];
+      const int k2 = pk[o * npx + px];
+      if (k2 >= 0 && (best < 0 || c2 < conf || (c2 == conf && k2 < best))) {
+        conf = c2;
+        best = k2;
+      }
     }
-    G(v->cost)[i * plane + p] = cv;
   }
+  if (part == 0 && best >= 0) L.win[px] = (uint32_t)best;
+  __syncthreads();
+  if (best >= 0) {
+    if (part == 0) {
+      const f4v h = ws.hyp(best, px);
+      G(v->conf)[p] = conf;
+      G(v->depth)[p] = h.w;
+      G(v->normal)[p] = h.x;
+      G(v->normal)[plane + p] = h.y;
+      G(v->normal)[2 * plane + p] = h.z;
+    }
+    for (int i = part; i < N; i += parts)
+      if ((sel >> i) & 1u) G(v->cost)[i * plane + p] = ws.M(best, i, px);
+  }
+  eval_unselected<R_, S_, STORE, RCP>(v, geo, L, ws, tile, ct, spl, R, v->compat_lo_geo_bug ? v->refInvK : v->refK, cnt);
   flush_counters(v, cnt);
 }
 
 template <int R_, int S_, int STORE, int RCP>
 __global__ __launch_bounds__(kSweepThreads) void k_local_opt(const LaunchTable* __restrict__ lt) {
-  __shared__ uint32_t tile[TileSize<R_>::kWords];
-  __shared__ float ct[256];
-  __shared__ float spl[SpSize<R_, S_>::kFloats];
+  __shared__ WinLds<R_, S_> lds;
+  __shared__ PassLds pass;
   __shared__ int next;
   for (int t = claim_tile(lt, &next); t >= 0; t = claim_tile(lt, &next))
-    local_opt_tile<R_, S_, STORE, RCP>(resolve(lt, t), tile, ct, spl);
+    local_opt_tile<R_, S_, STORE, RCP>(resolve(lt, t), lds, pass);
 }
 
 // Tiles of a launch of an element-wise phase, assigned by workgroup index
@@ -1702,6 +2029,10 @@ void* pick_kernel(const LaunchCfg& cfg) {
   return pick_sr<Kn, -1, -1>(cfg.storage, cfg.rcp);
 }
 
+bool compiled_window(const LaunchCfg& cfg) {
+  return (cfg.radius == 5 || cfg.radius == 7) && (cfg.step == 1 || cfg.step == 2);
+}
+
 }  // namespace
 
 
@@ -1750,23 +2081,38 @@ void* phase_kernel(PhaseKind kind, const LaunchCfg& cfg) {
   return nullptr;
 }
 
+// Launch-time LDS of a windowed phase whose window has no compiled kernel:
+// the spatial weights and the widest ref tile of the tile shapes.
+size_t window_lds_bytes(PhaseKind kind, const LaunchCfg& cfg) {
+  if (plain_phase(kind) || compiled_window(cfg)) return 0;
+  const int n = (2 * cfg.radius) / cfg.step + 1;
+  size_t words = 0;
+  for (int lw = kTileLog2WMin; lw <= kTileLog2WMax; ++lw) {
+    const size_t w = (size_t)((1 << lw) + 2 * cfg.radius) * ((kTilePixels >> lw) + 2 * cfg.radius);
+    words = w > words ? w : words;
+  }
+  return ((size_t)n * n + words) * sizeof(uint32_t);
+}
+
 }  // namespace
 
 namespace {
 std::mutex g_occ_mu;
-std::map<void*, int> g_occ;
+std::map<std::pair<void*, size_t>, int> g_occ;
 std::map<int, int> g_cus;
 }  // namespace
 
 int phase_occupancy(PhaseKind kind, const LaunchCfg& cfg) {
   void* fn = phase_kernel(kind, cfg);
   if (!fn) return 1;
+  const size_t dyn = window_lds_bytes(kind, cfg);
   std::lock_guard<std::mutex> lk(g_occ_mu);
-  auto it = g_occ.find(fn);
+  const std::pair<void*, size_t> key(fn, dyn);
+  auto it = g_occ.find(key);
   if (it == g_occ.end()) {
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, kSweepThreads, 0) != hipSuccess || n <= 0) n = 1;
-    it = g_occ.emplace(fn, n).first;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, kSweepThreads, dyn) != hipSuccess || n <= 0) n = 1;
+    it = g_occ.emplace(key, n).first;
   }
   return it->second;
 }
@@ -1793,12 +2139,24 @@ int phase_grid(PhaseKind kind, const LaunchCfg& cfg, int tiles, int blocks_per_c
   return (int)(g < tiles ? g : tiles);
 }
 
+// Tiles of 64 pixels (four waves on each) where tiles of 256 would not give
+// every workgroup slot of the chip one; above that the larger tile wins, since
+// its lists of 64 pairs are fuller.  Whole runs, 256 / 64 pixels:
+//   160x120  (38 of 1024 slots)    2.26 / 1.25 ms
+//   640x480  (600 of 1024)         6.60 / 6.21 ms
+//   1021x767 (1536 of 1024)        23.0 / 24.6 ms
+//   1920x1080 (4080 of 1024), geometric  78.1 / 78.2 ms
+bool small_tiles(PhaseKind kind, const LaunchCfg& cfg, int tiles, int blocks_per_cu) {
+  if (kind != kPhaseSweep && kind != kPhaseLocal) return false;
+  return tiles < phase_grid(kind, cfg, INT32_MAX, blocks_per_cu);
+}
+
 hipError_t launch_phase(PhaseKind kind, const LaunchCfg& cfg, const LaunchTable* table, int grid, hipStream_t s) {
   if (grid <= 0 || !table) return hipErrorInvalidValue;
   void* fn = phase_kernel(kind, cfg);
   if (!fn) return hipErrorInvalidValue;
   void* args[] = {(void*)&table};
-  return hipLaunchKernel(fn, dim3((unsigned)grid), dim3(kSweepThreads), args, 0, s);
+  return hipLaunchKernel(fn, dim3((unsigned)grid), dim3(kSweepThreads), args, window_lds_bytes(kind, cfg), s);
 }
 
 hipError_t launch_run_filter(const ViewDev* v, int W, int H, int dedup, float filter_max_cost, int min_consistent,

@@ -624,7 +624,7 @@ PM_API pm_status pm_server_create(pm_engine* e, const pm_server_config* cfg, pm_
   PM_HIP(hipSetDevice(e->device));
   int n_cu = 0;
   PM_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, e->device));
-  const size_t ws_floats = (size_t)n_cu * pm::kMaxBlocksPerCU * pm::kSweepThreads * pm::ws_floats_per_slot(PM_MAX_NUM_SRC);
+  const size_t ws_floats = (size_t)n_cu * pm::kMaxBlocksPerCU * pm::kSweepThreads * pm::ws_floats_per_pixel(PM_MAX_NUM_SRC);
   const size_t ws_bytes = Arena::round(ws_floats * sizeof(float));
   if (cfg->hbm_budget_bytes < ws_bytes + ((size_t)1 << 20))
     return fail(PM_ERR_OVER_BUDGET, "budget below the workspace reserve (" + std::to_string(ws_bytes) + " bytes)");

@@ -1,0 +1,73 @@
+"""The sweep and local optimisation list the evaluations that a tile needs and share them among a
+workgroup's waves.  Which evaluations are left out depends on the options, and the tile size on the
+launch; the maps are the transcription's bit for bit in every case."""
+import numpy as np
+import pytest
+
+from oracle import binding
+from sensemap_amd import abi, scene
+from sensemap_amd import patch_match as pmm
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    # more draws than a thread keeps in registers, weights by count
+    "counted_draws": (dict(num_samples=37, random_optimization=False), dict()),
+    "one_source": (dict(), dict(num_src=1)),
+    # costs near the largest float: a zero weight need not remove them, so nothing is left out
+    "unbounded_term": (dict(geom_consistency=True, geom_consistency_regularizer=1e38), dict()),
+    "geometric": (dict(geom_consistency=True), dict(num_src=7)),
+    # no source ever qualifies, and every source does
+    "none_good": (dict(num_good_hypothesis=12), dict()),
+    "all_good": (dict(num_good_hypothesis=0, num_bad_hypothesis=11), dict(num_src=6)),
+    "wide_runtime_window": (dict(window_radius=9, window_step=2), dict()),
+    "compensated": (dict(accum_mode=abi.PM_ACCUM_COMPENSATED, image_storage=abi.PM_STORAGE_U8), dict()),
+    # a tile's last row and column, fewer pixels than a wave
+    "edge": (dict(), dict(width=33, height=17)),
+    "sliver": (dict(window_radius=7, window_step=1), dict(width=129, height=3)),
+}
+
+
+def maps(v):
+    return {"depth": v.GetDepthMap(), "normal": v.GetNormalMap(), "conf": v.GetConfMap(),
+            "cost": v.GetCostMap(), "view_sel": v.GetViewSelMap()}
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_bitwise_alone_and_in_a_large_launch(name):
+    options, shape = CASES[name]
+    sc = scene.planes_scene(**dict(dict(seed=6, width=90, height=70, f=80.0, num_src=4), **shape))
+    opts = helpers.c1_options(num_iterations=4, **options)
+    prob = scene.to_problem(sc, with_gt_maps=opts.geom_consistency)
+    print(f"[shared] {name}", flush=True)
+    e = pmm.PatchMatchACMMCuda(opts, prob)
+    e.Run()
+    alone = maps(e)
+    cpu = binding.run_view(opts, e.view)
+    e.close()
+    assert not any(helpers.maps_equal(alone, cpu).values()), helpers.maps_equal(alone, cpu)
+    # beside a view of more tiles than the chip has workgroup slots: tiles of 256 pixels
+    big = scene.planes_scene(seed=7, width=1600, height=800, f=900.0, num_src=2)
+    rest = dict(options, geom_consistency=False, num_samples=15)
+    b = pmm.PatchMatchBatch([(opts, prob), (helpers.c1_options(num_iterations=4, **rest), scene.to_problem(big))])
+    b.Run()
+    together = maps(b.views[0])
+    b.close()
+    assert not any(helpers.maps_equal(together, alone).values()), helpers.maps_equal(together, alone)
+
+
+def test_a_counted_run_gives_the_same_maps():
+    # counting makes every evaluation of the algorithm, others leave out what cannot matter
+    sc = helpers.small_heightfield()
+    opts = helpers.c1_options(num_iterations=5, window_radius=7, window_step=1)
+    got = []
+    for counting in (False, True):
+        engine = pmm.Engine(0)
+        engine.set_counting(counting)
+        e = pmm.PatchMatchACMMCuda(opts, scene.to_problem(sc), engine=engine)
+        e.Run()
+        got.append(maps(e))
+        e.close()
+    assert not any(helpers.maps_equal(*got).values()), helpers.maps_equal(*got)
+    assert np.count_nonzero(got[0]["depth"]) > 0.9 * got[0]["depth"].size
