@@ -19,9 +19,6 @@ constexpr int kQuadPad = 4;          // zero texels around every source image
 constexpr int kTileLog2WMin = 4, kTileLog2WMax = 6, kTileLog2WDefault = 5;
 constexpr int kTilePixels = 512;
 constexpr int kTileLog2Px = 8;       // pixels of one colour in a tile: 256
-// The sweep and the local optimisation can also run on tiles of 16x8 pixels,
-// 64 of a colour, whose evaluations the workgroup's four waves share.
-constexpr int kSmallTileLog2W = 4, kSmallTileLog2Px = 6;
 constexpr int kMaxBlocksPerCU = 8;   // resident workgroups of a persistent launch per CU, at most
 constexpr int kSweepThreads = 256;
 constexpr float kMaxCost = 2.0f;
@@ -103,7 +100,7 @@ struct LaunchTable {
   int32_t total_tiles;   // tiles of the launch
   int32_t ws_stride;     // workspace floats per workgroup
   int32_t tile_lw;       // log2 of the tile width (kTileLog2WMin..kTileLog2WMax)
-  int32_t tile_lpx;      // log2 of a tile's pixels of one colour (kTileLog2Px or kSmallTileLog2Px)
+  int32_t tile_lpx;      // log2 of a tile's pixels of one colour (TileShape)
   int32_t pad0;
   float* ws;             // workspace of the launch
   uint32_t* queue;       // 8 tile counters (one per XCD range), zero at launch start
@@ -158,8 +155,12 @@ inline bool plain_phase(PhaseKind k) { return k >= kPhaseFilter; }
 // number of CUs times the workgroups one CU holds (capped by blocks_per_cu
 // when > 0), and never more than the tiles.
 int phase_grid(PhaseKind kind, const LaunchCfg& cfg, int tiles, int blocks_per_cu);
-// Whether a launch that would have `tiles` tiles of 256 pixels runs on tiles of 64.
-bool small_tiles(PhaseKind kind, const LaunchCfg& cfg, int tiles, int blocks_per_cu);
+// Tile of a launch over views of `pixels` pixels in all whose default or tuned
+// width is 2^lw: log2 of the width and of the pixels of one colour.
+struct TileShape {
+  int lw, lpx;
+};
+TileShape tile_shape(PhaseKind kind, const LaunchCfg& cfg, int lw, long long pixels, int blocks_per_cu);
 // Workgroups of the phase kernel one CU holds at once.
 int phase_occupancy(PhaseKind kind, const LaunchCfg& cfg);
 hipError_t launch_phase(PhaseKind kind, const LaunchCfg& cfg, const LaunchTable* table, int grid, hipStream_t s);

@@ -931,11 +931,11 @@ pm_status plan_launches(const std::vector<std::pair<pm_problem*, const std::vect
     }
   }
   for (Group& g : groups) {
-    pm_status rs = g.number_tiles(g.shape.tile_lw, pm::kTileLog2Px);
+    long long pixels = 0;
+    for (const pm_problem* p : g.views) pixels += (long long)p->W * p->H;
+    const pm::TileShape ts = pm::tile_shape(g.kind, g.cfg, g.shape.tile_lw, pixels, g.shape.blocks_per_cu);
+    pm_status rs = g.number_tiles(ts.lw, ts.lpx);
     if (rs != PM_OK) return rs;
-    if (pm::small_tiles(g.kind, g.cfg, g.tiles, g.shape.blocks_per_cu)) {
-      if ((rs = g.number_tiles(pm::kSmallTileLog2W, pm::kSmallTileLog2Px)) != PM_OK) return rs;
-    }
     const int grid = pm::phase_grid(g.kind, g.cfg, g.tiles, g.shape.blocks_per_cu);
     if (grid <= 0) return fail(PM_ERR_DEVICE, "no launch configuration for a phase kernel");
     const size_t off = (plan.tables.size() + 15) & ~(size_t)15;

@@ -1,7 +1,7 @@
 // pm_kernels.hip -- gfx950 kernels of the PatchMatch MVS engine.
 //
 // A 256-thread workgroup owns a 32x16 pixel tile (its 256 pixels of one
-// checkerboard colour), or a 16x8 one in small launches.  The sweep and the
+// checkerboard colour), or a 16x8 or 8x4 one in small launches.  The sweep and the
 // local optimisation list the (hypothesis, pixel) pairs that need a cost and
 // walk the windows of 64 pairs per wave; neighbouring pairs are neighbouring
 // pixels, so the windows of a wave overlap and their source footprints hit
@@ -72,15 +72,18 @@ __device__ __forceinline__ f4v ld_f4(const float4* p, int idx) {
 }
 
 __constant__ int c_neighbor_offs[4][2] = {{0, -1}, {-1, 0}, {0, 1}, {1, 0}};
-__constant__ int c_dir_samples[8][20] = {
-    {-1, -2, 1, -2, -2, -3, 2, -3, -3, -4, 3, -4, -4, -5, 4, -5, -5, -6, 5, -6},
-    {-1, 2, 1, 2, -2, 3, 2, 3, -3, 4, 3, 4, -4, 5, 4, 5, -5, 6, 5, 6},
-    {-2, -1, -2, 1, -3, -2, -3, 2, -4, -3, -4, 3, -5, -4, -5, 4, -6, -5, -6, 5},
-    {2, -1, 2, 1, 3, -2, 3, 2, 4, -3, 4, 3, 5, -4, 5, 4, 6, -5, 6, 5},
-    {0, -3, 0, -5, 0, -7, 0, -9, 0, -11, 0, -13, 0, -15, 0, -17, 0, -19, 0, -21},
-    {0, 3, 0, 5, 0, 7, 0, 9, 0, 11, 0, 13, 0, 15, 0, 17, 0, 19, 0, 21},
-    {-3, 0, -5, 0, -7, 0, -9, 0, -11, 0, -13, 0, -15, 0, -17, 0, -19, 0, -21, 0},
-    {3, 0, 5, 0, 7, 0, 9, 0, 11, 0, 13, 0, 15, 0, 17, 0, 19, 0, 21, 0}};
+// Sample f of direction gi (dirSamples, kernel_functions.cu): for gi < 4 the
+// wedge (-1, 2), (1, 2), (-2, 3), (2, 3) .. along its axis, for the others the
+// odd distances 3, 5 .. 21; the axis is the columns for gi & 2 == 0, the rows
+// otherwise, and points to smaller indices for even gi.  Computed, since the lanes of a wave
+// may take different directions.
+__device__ __forceinline__ void dir_sample(int gi, int sign, int f, int& dr, int& dc) {
+  const int m = f / 2 + 1;
+  const int along = sign * (gi < 4 ? m + 1 : 3 + 2 * f);
+  const int across = gi < 4 ? ((f & 1) ? m : -m) : 0;
+  dr = (gi & 2) ? along : across;
+  dc = (gi & 2) ? across : along;
+}
 __constant__ float c_mweights[5] = {0.f, 1.f, 2.01f, 3.03f, 4.06f};
 
 // ---------------------------------------------------------------------------
@@ -660,6 +663,7 @@ struct Ctx {
   int local_block;  // tile index within the view
   int lw;           // log2 of the tile width
   int lpx;          // log2 of the tile's pixels of one colour
+  int group;        // sources a step of eval_selected takes
   float* ws;        // this workgroup's workspace
 };
 
@@ -679,6 +683,12 @@ __device__ __forceinline__ Ctx resolve(const LaunchTable* __restrict__ lt, int t
   c.local_block = t - g->e[lo].tile_start;
   c.lw = g->tile_lw;
   c.lpx = g->tile_lpx;
+  // One source a step leaves out the most evaluations.  Small tiles have too
+  // few pairs of one source for four waves: two sources (640x480: 6.07 ms a
+  // run, against 6.25 with one and 6.21 with four), and four where every
+  // workgroup has one tile at most, so that the chain of steps is what counts
+  // (240x160: 2.33 ms, against 2.62 with two).
+  c.group = c.lpx == kTileLog2Px ? 1 : g->total_tiles <= (int)gridDim.x ? 4 : 2;
   c.ws = g->ws + (size_t)blockIdx.x * g->ws_stride;
   return c;
 }
@@ -1018,7 +1028,7 @@ __device__ __forceinline__ void eval_unselected(VPtr v, const Geo& geo, PassLds&
     int n = 0;
     for (int q0 = 0; q0 < ws.npx; q0 += 64) {
       const int q = q0 + lane;
-      const bool on = L.win[q] != kNone && !((L.sel[q] >> i) & 1u);
+      const bool on = q < ws.npx && L.win[q] != kNone && !((L.sel[q] >> i) & 1u);
       const uint64_t m = __ballot(on);
       if (on) own[n + rank_in(m)] = (uint8_t)q;
       n += __popcll(m);
@@ -1049,14 +1059,6 @@ __device__ __forceinline__ bool costs_bounded(VPtr v) {
 // ---------------------------------------------------------------------------
 // checkerboard sweep
 
-// Optional occupancy target for the sweep kernel (waves per SIMD), a build
-// knob for tuning register use against latency hiding.
-#ifdef PM_SWEEP_WAVES_PER_EU
-#define PM_SWEEP_OCC __attribute__((amdgpu_waves_per_eu(PM_SWEEP_WAVES_PER_EU, 8)))
-#else
-#define PM_SWEEP_OCC
-#endif
-
 // Samples of the CDF held in registers at a time.
 constexpr int kDraws = 16;
 
@@ -1070,7 +1072,7 @@ __device__ __forceinline__ void sweep_tile(const Ctx& cx, WinLds<R_, S_>& lds, P
   const int W = v->W, H = v->H, N = v->N;
   const int plane = W * H;
   const int npx = 1 << cx.lpx, parts = kSweepThreads >> cx.lpx;
-  const int px = threadIdx.x & (npx - 1), part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> cx.lpx));  // thread: a share of a pixel's bookkeeping
+  const int px = threadIdx.x & (npx - 1), part = threadIdx.x >> cx.lpx;  // thread: a share of a pixel's bookkeeping
   const int wave = wave_id(), lane = lane_id();
   const Geo geo = stage_tile(cx, R, tile_pitch<R_>(R, cx.lw), tile, lds.ct, spl);
   const Ws ws{cx.ws, npx, N};
@@ -1145,10 +1147,12 @@ __device__ __forceinline__ void sweep_tile(const Ctx& cx, WinLds<R_, S_>& lds, P
         const int gi = task - 1;
         float best_conf = PM_FLT_MAX;
         int br = 0, bc = 0;
+        const int sign = (gi & 1) ? 1 : -1;
 #pragma unroll
         for (int f = 0; f < 10; ++f) {
-          const int nr = row + c_dir_samples[gi][2 * f];
-          const int ncn = col + c_dir_samples[gi][2 * f + 1];
+          int dr, dc;
+          dir_sample(gi, sign, f, dr, dc);
+          const int nr = row + dr, ncn = col + dc;
           if (nr < 0 || nr >= H || ncn < 0 || ncn >= W) continue;
           const float cv = G(v->conf)[nr * W + ncn];
           if (best_conf > cv) {
@@ -1173,7 +1177,7 @@ __device__ __forceinline__ void sweep_tile(const Ctx& cx, WinLds<R_, S_>& lds, P
 
   // the candidates' pairs; then the cost matrix, source by source
   if (wave * 64 < npx) {
-    const uint32_t b = L.bits[wave * 64 + lane];
+    const uint32_t b = lane < npx ? L.bits[wave * 64 + lane] : 0u;
     int total = 0;
     for (int k = 1; k < kMaxHyp; ++k) total += __popcll(__ballot((b >> k) & 1u));
     int base = 0;
@@ -1350,7 +1354,7 @@ __device__ __forceinline__ void sweep_tile(const Ctx& cx, WinLds<R_, S_>& lds, P
   // not above rc0; only the selected sources enter that sum.
   float sum[kNumRefine - 1];
   const uint32_t alive = eval_selected<R_, S_, STORE, RCP, kNumRefine - 1>(
-      v, geo, L, ws, tile, ct, spl, R, px, part, parts, hb + 1, sel, full && sel != 0, full ? 1 : parts, sum, weight,
+      v, geo, L, ws, tile, ct, spl, R, px, part, parts, hb + 1, sel, full && sel != 0, full ? 1 : cx.group, sum, weight,
       [&](float s) __attribute__((always_inline)) { return s > rc0; },
       [&](int k, int i, int q, float m) __attribute__((always_inline)) { ws.RM(k + 1, i, q) = m; }, cnt);
   int b2 = -1;
@@ -1404,7 +1408,7 @@ __device__ __forceinline__ void sweep_tile(const Ctx& cx, WinLds<R_, S_>& lds, P
 }
 
 template <int R_, int S_, int STORE, int RCP>
-__global__ __launch_bounds__(kSweepThreads) PM_SWEEP_OCC void k_sweep(const LaunchTable* __restrict__ lt) {
+__global__ __launch_bounds__(kSweepThreads) void k_sweep(const LaunchTable* __restrict__ lt) {
   __shared__ WinLds<R_, S_> lds;
   __shared__ PassLds pass;
   __shared__ int next;
@@ -1425,7 +1429,7 @@ __device__ __forceinline__ void local_opt_tile(const Ctx& cx, WinLds<R_, S_>& ld
   const int W = v->W, H = v->H, N = v->N;
   const int plane = W * H;
   const int npx = 1 << cx.lpx, parts = kSweepThreads >> cx.lpx;
-  const int px = threadIdx.x & (npx - 1), part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> cx.lpx));
+  const int px = threadIdx.x & (npx - 1), part = threadIdx.x >> cx.lpx;
   const Geo geo = stage_tile(cx, R, tile_pitch<R_>(R, cx.lw), tile, lds.ct, spl);
   const Ws ws{cx.ws, npx, N};
   Counters cnt;
@@ -1484,7 +1488,7 @@ __device__ __forceinline__ void local_opt_tile(const Ctx& cx, WinLds<R_, S_>& ld
   const bool prune = !v->geom || v->geom_regularizer >= 0.0f;
   float sum[kLoTrials];
   const uint32_t alive = eval_selected<R_, S_, STORE, RCP, kLoTrials>(
-      v, geo, L, ws, tile, ct, spl, R, px, part, parts, 0, sel, false, v->counters != nullptr ? 1 : parts, sum,
+      v, geo, L, ws, tile, ct, spl, R, px, part, parts, 0, sel, false, v->counters != nullptr ? 1 : cx.group, sum,
       [](int) __attribute__((always_inline)) { return 1.0f; },
       [&](float s) __attribute__((always_inline)) { return prune && s / mw >= conf0; },
       [&](int k, int i, int q, float m) __attribute__((always_inline)) { ws.M(k, i, q) = m; }, cnt);
@@ -2139,16 +2143,22 @@ int phase_grid(PhaseKind kind, const LaunchCfg& cfg, int tiles, int blocks_per_c
   return (int)(g < tiles ? g : tiles);
 }
 
-// Tiles of 64 pixels (four waves on each) where tiles of 256 would not give
-// every workgroup slot of the chip one; above that the larger tile wins, since
-// its lists of 64 pairs are fuller.  Whole runs, 256 / 64 pixels:
-//   160x120  (38 of 1024 slots)    2.26 / 1.25 ms
-//   640x480  (600 of 1024)         6.60 / 6.21 ms
-//   1021x767 (1536 of 1024)        23.0 / 24.6 ms
-//   1920x1080 (4080 of 1024), geometric  78.1 / 78.2 ms
-bool small_tiles(PhaseKind kind, const LaunchCfg& cfg, int tiles, int blocks_per_cu) {
-  if (kind != kPhaseSweep && kind != kPhaseLocal) return false;
-  return tiles < phase_grid(kind, cfg, INT32_MAX, blocks_per_cu);
+// Tiles of 64 pixels of a colour (four waves on each) where tiles of 256 would
+// not give every workgroup slot of the chip one, and of 16 where those of 64
+// would leave CUs idle (a quarter of the slots: 4 workgroups to a CU).  Above
+// its line the larger tile wins: its lists of 64 pairs are fuller, and the
+// work that a workgroup does once per tile is spread further.  Whole runs in
+// ms, tiles of 256 / 64 / 16 pixels:
+//   96x64     4.22 / 1.79 / 1.25     160x120 (2 sources)  2.26 / 1.27 / 1.15
+//   240x160   4.50 / 2.33 / 2.87     640x480              6.58 / 6.25 / 12.9
+//   1021x767  23.0 / 24.6            1920x1080 geometric  78.1 / 78.2
+TileShape tile_shape(PhaseKind kind, const LaunchCfg& cfg, int lw, long long pixels, int blocks_per_cu) {
+  if (kind == kPhaseSweep || kind == kPhaseLocal) {
+    const long long slots = phase_grid(kind, cfg, INT32_MAX, blocks_per_cu);
+    if (pixels < slots / 4 * 128) return TileShape{3, 4};
+    if (pixels < slots * 512) return TileShape{4, 6};
+  }
+  return TileShape{lw, kTileLog2Px};
 }
 
 hipError_t launch_phase(PhaseKind kind, const LaunchCfg& cfg, const LaunchTable* table, int grid, hipStream_t s) {

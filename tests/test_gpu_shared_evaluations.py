@@ -47,14 +47,16 @@ def test_bitwise_alone_and_in_a_large_launch(name):
     cpu = binding.run_view(opts, e.view)
     e.close()
     assert not any(helpers.maps_equal(alone, cpu).values()), helpers.maps_equal(alone, cpu)
-    # beside a view of more tiles than the chip has workgroup slots: tiles of 256 pixels
-    big = scene.planes_scene(seed=7, width=1600, height=800, f=900.0, num_src=2)
-    rest = dict(options, geom_consistency=False, num_samples=15)
-    b = pmm.PatchMatchBatch([(opts, prob), (helpers.c1_options(num_iterations=4, **rest), scene.to_problem(big))])
-    b.Run()
-    together = maps(b.views[0])
-    b.close()
-    assert not any(helpers.maps_equal(together, alone).values()), helpers.maps_equal(together, alone)
+    # alone it runs on tiles of 16 pixels; beside a larger view on tiles of 64, and beside one of more
+    # tiles than the chip has workgroup slots on tiles of 256
+    for width, height in ((480, 320), (1600, 800)):
+        big = scene.planes_scene(seed=7, width=width, height=height, f=900.0, num_src=2)
+        rest = dict(options, geom_consistency=False, num_samples=15)
+        b = pmm.PatchMatchBatch([(opts, prob), (helpers.c1_options(num_iterations=4, **rest), scene.to_problem(big))])
+        b.Run()
+        together = maps(b.views[0])
+        b.close()
+        assert not any(helpers.maps_equal(together, alone).values()), helpers.maps_equal(together, alone)
 
 
 def test_a_counted_run_gives_the_same_maps():
