@@ -28,8 +28,8 @@
 //     wave that finishes that predecessor runs the first walk it made ready
 //     itself and puts the others in a ready queue, from which the other
 //     waves take them.  A wave replays its walk over the graph (the whole
-//     wave: the set of available nodes in scalar registers, one lane per
-//     push), sets the accepted pixels' mask bits, publishes them with a
+//     wave; nodes that earlier walks took are left out first, and up to 64
+//     others are replayed from registers), sets the accepted pixels' mask bits, publishes them with a
 //     release fence and counts itself off at each successor.  Everything a
 //     wave reads that another wrote (queue slots, mask words) is an
 //     agent-scope atomic load, since the waves run on every XCD.  A wave
@@ -66,15 +66,19 @@ constexpr int kProvChild = 4096;                  // push slots met building a g
 constexpr int kHash = 1024;                       // open-addressing slots (gid -> pixel)
 constexpr int64_t kMaxWindow = int64_t(1) << 23;  // seeds per window
 // Build knobs of the dataflow, defaults measured on the 1920x1080 11-view
-// scene (8: one wave per CU; 16 s_sleep units between polls).
+// scene (8: one wave per CU; 32 s_sleep units between polls).
 #ifndef PM_FLOW_WAVES_PER_8CU
 #define PM_FLOW_WAVES_PER_8CU 8
 #endif
 constexpr int kFlowWavesPer8CU = PM_FLOW_WAVES_PER_8CU;  // dataflow waves per 8 CUs
 #ifndef PM_POLL_SLEEP
-#define PM_POLL_SLEEP 16
+#define PM_POLL_SLEEP 32
 #endif
-constexpr int kPollSleep = PM_POLL_SLEEP;  // s_sleep units (64 clocks) between polls of a queue slot
+// s_sleep units (64 clocks) between polls of a queue slot.  The polls of the
+// waiting waves slow the running walks more than a longer sleep delays a
+// walk's start: whole calls with 8, 16, 32 and 64 units took 462, 452, 440 and
+// 441 ms (1920x1080, 11 views) and 55, 51, 48 and 49 ms (640x480, 5 views).
+constexpr int kPollSleep = PM_POLL_SLEEP;
 constexpr int kPollCheck = 64;             // polls between looks at the shared counters
 constexpr double kWaitSeconds = 4.0;  // one wait's bound
 
@@ -715,6 +719,13 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(const int32_t* __re
     }
 }
 
+// What the dataflow needs of a walk before its graph, in one record: taken
+// from the arrays it is gathered from, it is seven reads in seven places.
+struct __attribute__((aligned(16))) Head {
+  int32_t nn, nch, np, ns;  // nodes, pushes, predecessors, successors
+  int32_t no, co, se, pad;  // first node, first push, end of the successor list
+};
+
 // The dataflow's state, for one segment of a window's walks (the window's
 // walks between two that run alone).
 struct Flow {
@@ -729,6 +740,7 @@ struct Flow {
   int32_t* nsucc;          // [seed] later walks that depend on it
   int32_t* succ_end;       // [seed] end of its successor list (the prefix sum, advanced by the scatter)
   int32_t* succ;           // successor lists
+  Head* head;              // [seed]
   int32_t* depth;          // [seed] 1 + the longest chain of walks it depends on
   int32_t* res_cnt;        // [seed] pixels accepted
   int16_t* res_nodes;      // [node] accepted nodes in visiting order, at the graph's node offset
@@ -841,6 +853,64 @@ __device__ __attribute__((always_inline)) inline int replay(const FusParams& prm
   return na;
 }
 
+// The same walk where at most 64 nodes are available (nearly always: of a
+// graph's nodes, earlier walks have taken most).  Nodes are numbered by rank
+// among the available ones; lane r holds node r's pushes of available nodes,
+// the last push lowest, kPackBits bits each, and their set.
+// No stack is kept: what is available was never popped, so the topmost entry
+// that would not be skipped is the last available push of the node taken last
+// among those that have one.  Lane j holds the set and pushes of the j-th
+// taken node, and a step is one ballot over them, without LDS.  The replays
+// of a row of seeds run one after another, so the instructions of a step
+// count: about 40, where the stack takes 150.
+// Returns the count; lane j gets the rank of the j-th taken node.
+constexpr int kPackBits = 6, kPackMax = 64 / kPackBits;
+
+__device__ __forceinline__ uint64_t lane_u64(uint64_t x, int l) {
+  return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, l) |
+         ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), l) << 32);
+}
+
+__device__ __forceinline__ int replay_ranked(uint64_t avail, uint64_t set, uint64_t pushes, int& taken) {
+  const int lane = threadIdx.x % 64;
+  const int shift = kPackBits * lane;
+  uint64_t tset = 0, tpushes = 0;
+  int na = 0, cur = 0;
+  taken = 0;
+  for (;;) {
+    avail &= ~(1ull << cur);
+    const uint64_t cset = lane_u64(set, cur);
+    uint64_t list = lane_u64(pushes, cur);
+    if (lane == na) {
+      tset = cset;
+      tpushes = list;
+      taken = cur;
+    }
+    ++na;
+    if (!(cset & avail)) {
+      const uint64_t m = __ballot((tset & avail) != 0);
+      if (!m) break;
+      list = lane_u64(tpushes, 63 - __clzll((long long)m));
+    }
+    // entries past the last are 0, the seed, which is taken
+    const uint64_t m = __ballot(lane < kPackMax && ((avail >> ((list >> shift) & 63u)) & 1u));
+    cur = (int)((list >> (kPackBits * (__ffsll((long long)m) - 1))) & 63u);
+  }
+  return na;
+}
+
+// Maximum over the wave, in every lane.
+__device__ __forceinline__ int wave_max(int x) {
+#define PM_DPP_MAX(ctrl) x = max(x, __builtin_amdgcn_update_dpp(x, x, ctrl, 0xf, 0xf, false))
+  PM_DPP_MAX(0x111);  // row_shr 1, 2, 4, 8: each row's maximum in its last lane
+  PM_DPP_MAX(0x112);
+  PM_DPP_MAX(0x114);
+  PM_DPP_MAX(0x118);
+#undef PM_DPP_MAX
+  return max(max(__builtin_amdgcn_readlane(x, 15), __builtin_amdgcn_readlane(x, 31)),
+             max(__builtin_amdgcn_readlane(x, 47), __builtin_amdgcn_readlane(x, 63)));
+}
+
 __device__ inline bool masked_now(const uint32_t* mask, int64_t gid) {
   return (__hip_atomic_load(mask + (gid >> 5), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> (gid & 31)) & 1u;
 }
@@ -904,6 +974,20 @@ __global__ void __launch_bounds__(256) k_succ(Pool g, Flow f) {
   if (np == 0) f.queue[atomicAdd(f.counters + 1, 1)] = ws;
 }
 
+// The walks' records, once their successor lists have their places.
+__global__ void __launch_bounds__(256) k_heads(Pool g, Flow f) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= f.n_tickets) return;
+  const int ws = f.tickets[t];
+  f.head[ws] = Head{g.n[ws], g.nc[ws], f.npred[ws], f.nsucc[ws], g.node_off[ws], g.child_off[ws], f.succ_end[ws], 0};
+}
+
+__device__ __forceinline__ Head load_head(const Flow& f, int ws) {
+  const int4* r = (const int4*)(f.head + ws);
+  const int4 a = r[0], b = r[1];
+  return Head{a.x, a.y, a.z, a.w, b.x, b.y, b.z, 0};
+}
+
 // The dataflow: persistent waves take queue slots in order; a slot's walk is
 // written once all the walks it depends on have finished.  A wave replays
 // its walk over the graph against the masks, sets the accepted pixels' mask
@@ -915,6 +999,13 @@ __global__ void __launch_bounds__(256) k_succ(Pool g, Flow f) {
 // the wave that made it ready or written to a slot, so a wave waiting on a
 // slot gets a walk or sees every walk finished; it gives up only when no walk
 // anywhere finished for wait_ticks.
+// Bound by latency: a wave is alone on its CU, and a walk is a chain of about
+// five round trips to memory that other XCDs write (about 2000 clocks each)
+// and the replay.  Clocks per walk before and after the replay from registers,
+// the records (Head) with the likely next one loaded ahead, and the statistic
+// taken off the chain: up to the masks 6700 / 5900 (of it the predecessors'
+// depths 2000 / 0), replay 9600 / 5400, after it 3100 / 3300; k_flow 201 / 165
+// ms a call at 1920x1080 with 11 views, 24.9 / 18 ms at 640x480 with 5.
 __global__ void __launch_bounds__(64) k_flow(FusParams prm, Pool g, uint32_t* mask, Flow f) {
   __shared__ __attribute__((aligned(16))) int64_t ngid[kNodeCap];
   __shared__ __attribute__((aligned(16))) int16_t nbase[kNodeCap];
@@ -922,7 +1013,11 @@ __global__ void __launch_bounds__(64) k_flow(FusParams prm, Pool g, uint32_t* ma
   __shared__ __attribute__((aligned(16))) int16_t child[kChildCap];
   __shared__ int32_t stack[kChildCap + 1];
   __shared__ int16_t accl[kNodeCap];
+  __shared__ uint8_t rank[kNodeCap];  // of an available node among them; 0xff otherwise
+  __shared__ uint8_t ranked[64];      // the available nodes by rank
   const int lane = threadIdx.x;
+  Head ahead{};         // of walk ahead_ws: the successor loaded while its predecessor was replayed
+  int ahead_ws = -1;
   int next = -1;  // a walk this wave made ready and runs next, past the queue (wave-uniform)
   for (;;) {
     int ws = next;
@@ -960,16 +1055,15 @@ __global__ void __launch_bounds__(64) k_flow(FusParams prm, Pool g, uint32_t* ma
     ws = __builtin_amdgcn_readfirstlane(ws);
     if (ws < 0) break;  // stopped, or every walk finished
     }
-    const int nn = g.n[ws], nch = g.nc[ws];
-    const int64_t no = g.node_off[ws], co = g.child_off[ws];
-    const int np = f.npred[ws], ns = f.nsucc[ws], se = f.succ_end[ws];
-    // what the end of the walk needs, loaded early: the longest chain behind
-    // it (a statistic: a predecessor's depth is stored without ordering
-    // against its countdown and may still read as the segment's 0, so the
-    // chain counted is a lower bound) and its successors
-    int dep = 0;
-    for (int k = lane; k < np; k += 64)
-      dep = max(dep, __hip_atomic_load(f.depth + f.preds[no + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    const Head head = ws == ahead_ws ? ahead : load_head(f, ws);
+    const int nn = head.nn, nch = head.nch, np = head.np, ns = head.ns, se = head.se;
+    const int64_t no = head.no, co = head.co;
+    // the first predecessors, for the longest chain behind the walk (a
+    // statistic: a predecessor's depth is stored without ordering against its
+    // countdown and may still read as the segment's 0, so the chain counted
+    // is a lower bound); nothing waits for them before the walk's end
+    const int pr0 = lane < np ? f.preds[no + lane] : -1;
+    // its successors, which the end of the walk needs
     const int sw0 = lane < ns ? f.succ[se - ns + lane] : -1;
     // the graph into LDS, every load in flight at once and together with
     // the seed's mask word: a graph's nodes and pushes start at multiples of
@@ -1001,6 +1095,12 @@ __global__ void __launch_bounds__(64) k_flow(FusParams prm, Pool g, uint32_t* ma
     if (lh1) *(uint4*)(child + 8 * (64 + lane)) = h1;
     if (lh2) *(uint4*)(child + 8 * (128 + lane)) = h2;
     if (lh3) *(uint4*)(child + 8 * (192 + lane)) = h3;
+    // The next walk on the chain is most often the right-hand neighbour's:
+    // its header is loaded beside this walk's masks.
+    const uint64_t right = __ballot(sw0 == ws + 1);
+    ahead_ws = ns > 0 ? (right ? ws + 1 : __builtin_amdgcn_readfirstlane(sw0)) : -1;
+    if (ahead_ws >= 0) ahead = load_head(f, ahead_ws);
+    int dep = pr0 >= 0 ? __hip_atomic_load(f.depth + pr0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
     int na = 0;
     if (seed_free) {
       __builtin_amdgcn_wave_barrier();
@@ -1019,7 +1119,50 @@ __global__ void __launch_bounds__(64) k_flow(FusParams prm, Pool g, uint32_t* ma
       ok.w1 = __ballot(64 + lane < nn && !m1);
       ok.w2 = __ballot(128 + lane < nn && !m2);
       ok.w3 = __ballot(192 + lane < nn && !m3);
-      na = replay(prm, ok, info, child, stack, accl);
+      const int nav = __popcll(ok.w0) + __popcll(ok.w1) + __popcll(ok.w2) + __popcll(ok.w3);
+      // no cut by depth or count can happen within nav nodes
+      bool ranks = (ok.w0 & 1ull) && nav <= 64 && nav < prm.max_traversal && nav <= prm.max_num_pixels;
+      uint64_t set = 0, pushes = 0;
+      if (ranks) {
+        const uint64_t lt = (1ull << lane) - 1;
+        int before = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint64_t w = r == 0 ? ok.w0 : r == 1 ? ok.w1 : r == 2 ? ok.w2 : ok.w3;
+          if (64 * r < nn) {
+            const bool a = (w >> lane) & 1ull;
+            const int k = before + __popcll(w & lt);
+            rank[64 * r + lane] = a ? (uint8_t)k : (uint8_t)0xff;
+            if (a) ranked[k] = (uint8_t)(64 * r + lane);
+            before += __popcll(w);
+          }
+        }
+        __builtin_amdgcn_wave_barrier();
+        int first = 0, cnt = 0;
+        if (lane < nav) {
+          const int node = ranked[lane];
+          first = nbase[node];
+          cnt = first >= 0 ? ncnt[node] : 0;
+        }
+        int packed = 0;
+        const int most = wave_max(cnt);
+        for (int k = 0; k < most; ++k) {
+          const int r = k < cnt ? rank[child[first + k]] : 0xff;
+          if (r != 0xff) {
+            set |= 1ull << r;
+            pushes = (pushes << kPackBits) | (uint64_t)r;
+            ++packed;
+          }
+        }
+        ranks = !__any(packed > kPackMax);
+      }
+      if (ranks) {
+        int taken;
+        na = replay_ranked(nav == 64 ? ~0ull : (1ull << nav) - 1, set, pushes, taken);
+        if (lane < na) accl[lane] = ranked[taken];
+      } else {
+        na = replay(prm, ok, info, child, stack, accl);
+      }
       __builtin_amdgcn_wave_barrier();
       for (int j = lane; j < na; j += 64) {
         const int node = accl[j];
@@ -1039,14 +1182,17 @@ __global__ void __launch_bounds__(64) k_flow(FusParams prm, Pool g, uint32_t* ma
       const int sw = k0 == 0 ? sw0 : (k0 + lane < ns ? f.succ[se - ns + k0 + lane] : -1);
       const bool ready = sw >= 0 && atomicSub(f.pending + sw, 1) == 1;
       const uint64_t rm = __ballot(ready);
-      const int kl = next < 0 && rm ? __ffsll((long long)rm) - 1 : -1;
+      const uint64_t pm = rm & __ballot(sw == ahead_ws);  // the one loaded ahead, if it is ready
+      const int kl = next < 0 && rm ? __ffsll((long long)(pm ? pm : rm)) - 1 : -1;
       if (ready && lane != kl)
         __hip_atomic_store(f.queue + atomicAdd(f.counters + 1, 1), sw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (kl >= 0) next = __builtin_amdgcn_readlane(sw, kl);
     }
     // the statistic after the countdown: its loads are then waited for
     // together with the countdown's, not before it
-    for (int d = 32; d > 0; d >>= 1) dep = max(dep, __shfl_xor(dep, d));
+    for (int k = 64 + lane; k < np; k += 64)
+      dep = max(dep, __hip_atomic_load(f.depth + f.preds[no + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    dep = wave_max(dep);
     if (lane == 0) {
       f.res_cnt[ws] = na;
       __hip_atomic_store(f.depth + ws, dep + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1625,6 +1771,8 @@ PM_API pm_status pm_fusion_run(pm_engine* e, const pm_fusion_options* o, int32_t
   f.nsucc = w_nsucc.as<int32_t>();
   f.succ_end = w_succend.as<int32_t>();
   f.succ = w_succ.as<int32_t>();
+  static_assert(sizeof(Head) <= sizeof(PointRec), "the records lie in the points' buffer until the points are formed");
+  f.head = w_out.as<Head>();
   f.depth = w_depth.as<int32_t>();
   f.res_cnt = w_rescnt.as<int32_t>();
   f.res_nodes = w_resnodes.as<int16_t>();
@@ -1738,6 +1886,7 @@ PM_API pm_status pm_fusion_run(pm_engine* e, const pm_fusion_options* o, int32_t
           hipLaunchKernelGGL(k_preds, dim3((nts + kPredWaves - 1) / kPredWaves), dim3(64 * kPredWaves), 0, st, g, fs);
           scan(f.nsucc + fs.seg_lo, f.succ_end + fs.seg_lo, span, w_sums.as<int32_t>(), w_total.as<int32_t>(), st);
           hipLaunchKernelGGL(k_succ, dim3((nts + 255) / 256), dim3(256), 0, st, g, fs);
+          hipLaunchKernelGGL(k_heads, dim3((nts + 255) / 256), dim3(256), 0, st, g, fs);
           hipLaunchKernelGGL(k_flow, dim3(std::min<unsigned>(flow_grid, (unsigned)nts)), dim3(64), 0, st, prm, g,
                              mask, fs);
           hipLaunchKernelGGL(k_segment_end, dim3(1), dim3(1), 0, st, (const int32_t*)f.counters,

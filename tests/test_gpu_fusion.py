@@ -131,3 +131,22 @@ def test_grey_and_three_channel_images_equal_transcription():
     print("[fusion] grey vs three channels: points", len(grey["score"]), flush=True)
     same(grey, col)
     same(grey, binding.fusion(ims, o))
+
+
+@pytest.mark.parametrize("options", [
+    dict(),                                          # a seed's walk meets a few free nodes: replayed from registers
+    dict(max_traversal_depth=4),                     # cut by depth: from the stack
+    dict(max_num_pixels=7),                          # cut by count
+    dict(max_depth_error=0.2, max_reproj_error=12.0, max_normal_error=60.0),  # more than 64 free nodes
+    dict(step_size=1, min_num_pixels=2),
+])
+@pytest.mark.parametrize("pushes", [3, 14])          # up to 10 of a node's pushes fit a lane's registers
+def test_replays_equal_transcription(pushes, options):
+    images = orbit_images(cams=15, nbr=pushes)
+    if pushes > 6:
+        for k, im in enumerate(images):
+            im.overlapping = [(k + s) % 15 for s in range(1, 15)]
+    got, want = fuse(images, StereoFusionOptions(**options)), binding.fusion(images, StereoFusionOptions(**options))
+    print("[fusion] replay", pushes, options, "points", len(got["score"]), flush=True)
+    assert len(want["score"]) > 0
+    same(got, want)
