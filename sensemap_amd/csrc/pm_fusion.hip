@@ -79,6 +79,7 @@ constexpr int kFlowWavesPer8CU = PM_FLOW_WAVES_PER_8CU;  // dataflow waves per 8
 // walk's start: whole calls with 8, 16, 32 and 64 units took 462, 452, 440 and
 // 441 ms (1920x1080, 11 views) and 55, 51, 48 and 49 ms (640x480, 5 views).
 constexpr int kPollSleep = PM_POLL_SLEEP;
+constexpr int kFinishedBatch = 32;         // walks a wave finishes before it says so, if it need not wait
 constexpr int kPollCheck = 64;             // polls between looks at the shared counters
 constexpr double kWaitSeconds = 4.0;  // one wait's bound
 
@@ -299,7 +300,7 @@ struct Pool {
   int16_t* cbase;      // [node] first push within the graph's; -1 when not expanded
   int16_t* ccnt;       // [node] pushes
   int16_t* child;      // [push] node index
-  unsigned long long* used;  // [2] nodes and pushes handed out
+  unsigned long long* used;  // handed out, in units of 8: nodes in the low half, pushes in the high
   int32_t* no_room;          // first seed of the window that found no room
   int64_t node_cap, child_cap;
 };
@@ -325,7 +326,9 @@ __global__ void __launch_bounds__(64) k_graph(const FusImgDev* __restrict__ imgs
   const int ws = blockIdx.x, lane = threadIdx.x;
   if (ws >= count) return;
   // past a seed that found the pool full: no room either (that seed ends the window)
-  if (ws > __hip_atomic_load(g.no_room, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+  // (a stale value only costs the build: what the window holds is decided by
+  // the final one)
+  if (ws > __hip_atomic_load(g.no_room, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) {
     if (lane == 0) g.n[ws] = -2;
     return;
   }
@@ -577,8 +580,12 @@ __global__ void __launch_bounds__(64) k_graph(const FusImgDev* __restrict__ imgs
     // nodes and pushes start at multiples of 8 elements (k_flow loads them
     // 16 bytes at a time)
     const unsigned long long np8 = (unsigned long long)((np + 7) & ~7), nc8 = (unsigned long long)((nch2 + 7) & ~7);
-    const unsigned long long no = atomicAdd(g.used, np8);
-    const unsigned long long co = atomicAdd(g.used + 1, nc8);
+    // one atomic for both: every seed's goes to the same address (with the
+    // cached look at no_room, k_graph 179 / 166 ms a call, 11 views of
+    // 1920x1080).  A window's seeds (kMaxWindow) times the largest graph fit
+    // the halves.
+    const unsigned long long at = atomicAdd(g.used, (np8 >> 3) | (nc8 >> 3 << 32));
+    const unsigned long long no = (at & 0xffffffffull) << 3, co = at >> 32 << 3;
     if (no + np8 > (unsigned long long)g.node_cap || co + nc8 > (unsigned long long)g.child_cap) {
       offs[0] = -1;
       atomicMin(g.no_room, ws);
@@ -741,6 +748,7 @@ struct Flow {
   int32_t* succ_end;       // [seed] end of its successor list (the prefix sum, advanced by the scatter)
   int32_t* succ;           // successor lists
   Head* head;              // [seed]
+  unsigned long long* kept;  // walks that accepted pixels, over the call
   int32_t* depth;          // [seed] 1 + the longest chain of walks it depends on
   int32_t* res_cnt;        // [seed] pixels accepted
   int16_t* res_nodes;      // [node] accepted nodes in visiting order, at the graph's node offset
@@ -1018,10 +1026,18 @@ __global__ void __launch_bounds__(64) k_flow(FusParams prm, Pool g, uint32_t* ma
   const int lane = threadIdx.x;
   Head ahead{};         // of walk ahead_ws: the successor loaded while its predecessor was replayed
   int ahead_ws = -1;
+  // This wave's walks, added up: the counters are one cache line for every
+  // wave, and an atomic a walk on it delayed the walks' own (k_flow 165 ms a
+  // call with the longest chain's, 134 without it; 11 views of 1920x1080).
+  int kept = 0, longest = 0, finished = 0;
   int next = -1;  // a walk this wave made ready and runs next, past the queue (wave-uniform)
   for (;;) {
     int ws = next;
     next = -1;
+    if (finished > 0 && (ws < 0 || finished >= kFinishedBatch)) {  // before it may wait, and now and then
+      if (lane == 0) atomicAdd(f.counters + 2, finished);
+      finished = 0;
+    }
     if (ws < 0) {
     // the slot: every lane takes part in the atomic (only lane 0 adds), the
     // result is wave-uniform.  A lane-0-only branch here lets the compiler
@@ -1196,9 +1212,14 @@ __global__ void __launch_bounds__(64) k_flow(FusParams prm, Pool g, uint32_t* ma
     if (lane == 0) {
       f.res_cnt[ws] = na;
       __hip_atomic_store(f.depth + ws, dep + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      atomicMax(f.counters + 4, dep + 1);
     }
-    if (lane == 0) atomicAdd(f.counters + 2, 1);
+    kept += na > 0 ? 1 : 0;
+    longest = max(longest, dep + 1);
+    ++finished;
+  }
+  if (lane == 0 && longest > 0) {
+    atomicMax(f.counters + 4, longest);
+    atomicAdd(f.kept, (unsigned long long)kept);
   }
 }
 
@@ -1223,7 +1244,12 @@ __global__ void __launch_bounds__(256) k_commit_alone(const WalkRec* __restrict_
 constexpr int kPtWaves = 2;
 constexpr int kLdsAcc = kNodeCap;           // accepted pixels staged in LDS per wave
 constexpr int kMaxImages = 65536;           // fusion takes at most this many images
-constexpr int kImgWords = kMaxImages / 32;  // visibility bitmap per wave
+// Visibility bitmaps, one per wave: launch-time LDS, sized by the call's
+// images (at kMaxImages it would be 8 KB a wave, and 8 waves to a CU).  With
+// the lane prefix in log steps: k_points 31 / 7.4 ms a call (11 views of
+// 1920x1080).
+extern __shared__ uint32_t image_bits[];
+inline size_t image_bits_bytes(int n_images) { return (size_t)kPtWaves * ((n_images + 31) / 32) * sizeof(uint32_t); }
 
 __device__ inline float pick(bool c0, float x0, bool c1, float x1) {
   const uint64_t m0 = __ballot(c0), m1 = __ballot(c1);
@@ -1318,12 +1344,12 @@ __device__ bool form_point(bool active, int na, const Src& src, const FusParams&
   const int k0 = min(lane * per, words), k1 = min(k0 + per, words);
   int mine = 0;
   for (int k = k0; k < k1; ++k) mine += __popc(bits[k]);
-  int before = 0, nvis = 0;
-  for (int l = 0; l < 64; ++l) {
-    const int c = __shfl(mine, l);
-    before += l < lane ? c : 0;
-    nvis += c;
+  int upto = mine;  // inclusive prefix over the lanes
+  for (int d = 1; d < 64; d <<= 1) {
+    const int t = __shfl_up(upto, d);
+    if (lane >= d) upto += t;
   }
+  const int before = upto - mine, nvis = __builtin_amdgcn_readlane(upto, 63);
   if (nvis < prm.min_num_visible) return false;
   PointRec r{};
   r.nvis = nvis;
@@ -1378,15 +1404,13 @@ __device__ bool form_point(bool active, int na, const Src& src, const FusParams&
 __global__ void __launch_bounds__(64 * kPtWaves) k_points(const FusImgDev* __restrict__ imgs, FusParams prm,
                                                           int32_t window_first, Pool g, Flow f,
                                                           PointRec* __restrict__ pts, int32_t* __restrict__ has,
-                                                          int32_t* __restrict__ vis_pool,
-                                                          unsigned long long* __restrict__ kept) {
+                                                          int32_t* __restrict__ vis_pool) {
   __shared__ float lv[kPtWaves][kVals][kLdsAcc];
-  __shared__ uint32_t bits[kPtWaves][kImgWords];
+  uint32_t* bits = image_bits + threadIdx.x / 64 * ((prm.n_images + 31) / 32);
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int t = blockIdx.x * kPtWaves + wave;
   const int ws = __builtin_amdgcn_readfirstlane(t < f.n_tickets ? f.tickets[t] : 0);
   const int na = __builtin_amdgcn_readfirstlane(t < f.n_tickets ? f.res_cnt[ws] : 0);
-  if (lane == 0 && na > 0) atomicAdd(kept, 1ull);
   const bool active = na >= prm.min_num_pixels;
   const int64_t no = active ? g.node_off[ws] : 0;
   GraphSrc src{imgs, g.gid, g.img, f.res_nodes, no, &prm, {0, 0, 0}, {0, 0, 0}};
@@ -1400,7 +1424,7 @@ __global__ void __launch_bounds__(64 * kPtWaves) k_points(const FusImgDev* __res
       src.ref_n[k] = v[3 + k];
     }
   }
-  if (form_point(active, na, src, prm, lv[wave], bits[wave], pts + ws, vis_pool + no) && lane == 0) has[ws] = 1;
+  if (form_point(active, na, src, prm, lv[wave], bits, pts + ws, vis_pool + no) && lane == 0) has[ws] = 1;
 }
 
 // The point of a walk run alone (the block's first wave).
@@ -1409,12 +1433,12 @@ __global__ void __launch_bounds__(64 * kPtWaves) k_points_alone(FusParams prm, c
                                                                 PointRec* __restrict__ out, int32_t* __restrict__ has,
                                                                 int32_t* __restrict__ vis_out) {
   __shared__ float lv[kPtWaves][kVals][kLdsAcc];
-  __shared__ uint32_t bits[kPtWaves][kImgWords];
+  uint32_t* bits = image_bits + threadIdx.x / 64 * ((prm.n_images + 31) / 32);
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int na = __builtin_amdgcn_readfirstlane(wave == 0 ? rec->n_acc : 0);
   const bool active = wave == 0 && na >= prm.min_num_pixels;
   const AccSrc src{acc};
-  const bool made = form_point(active, na, src, prm, lv[wave], bits[wave], out, vis_out);
+  const bool made = form_point(active, na, src, prm, lv[wave], bits, out, vis_out);
   if (wave == 0 && lane == 0) *has = made ? 1 : 0;
 }
 
@@ -1478,7 +1502,7 @@ __global__ void __launch_bounds__(256) k_fill_u32(uint32_t* __restrict__ p, int6
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = 0u;
 }
 __global__ void k_window_reset(unsigned long long* used, int32_t* no_room, int32_t count, int32_t* status) {
-  used[0] = used[1] = 0ull;
+  *used = 0ull;
   *no_room = count;
   status[0] = status[1] = status[2] = 0;
 }
@@ -1714,7 +1738,7 @@ PM_API pm_status pm_fusion_run(pm_engine* e, const pm_fusion_options* o, int32_t
   if (pm_status s = p_cbase.get(nd_b * 2)) return s;
   if (pm_status s = p_ccnt.get(nd_b * 2)) return s;
   if (pm_status s = p_child.get((size_t)child_cap * 2)) return s;
-  if (pm_status s = p_used.get(16)) return s;
+  if (pm_status s = p_used.get(8)) return s;
   if (pm_status s = p_room.get(4)) return s;
   if (pm_status s = w_cnt.get((size_t)total * 4)) return s;
   if (pm_status s = w_end.get((size_t)total * 4)) return s;
@@ -1771,8 +1795,10 @@ PM_API pm_status pm_fusion_run(pm_engine* e, const pm_fusion_options* o, int32_t
   f.nsucc = w_nsucc.as<int32_t>();
   f.succ_end = w_succend.as<int32_t>();
   f.succ = w_succ.as<int32_t>();
+  static_assert(kMaxWindow * kChildCap / 8 < (int64_t(1) << 32), "the pool's reservations");
   static_assert(sizeof(Head) <= sizeof(PointRec), "the records lie in the points' buffer until the points are formed");
   f.head = w_out.as<Head>();
+  f.kept = w_kept.as<unsigned long long>();
   f.depth = w_depth.as<int32_t>();
   f.res_cnt = w_rescnt.as<int32_t>();
   f.res_nodes = w_resnodes.as<int16_t>();
@@ -1914,7 +1940,7 @@ PM_API pm_status pm_fusion_run(pm_engine* e, const pm_fusion_options* o, int32_t
                            b_gids.as<int64_t>(), b_acc.as<AccEntry>(), b_stack.as<StackEntry>());
         hipLaunchKernelGGL(k_commit_alone, dim3(fill_grid(big_acc)), dim3(256), 0, st, (const WalkRec*)b_rec.p,
                            (const int64_t*)b_gids.p, mask);
-        hipLaunchKernelGGL(k_points_alone, dim3(1), dim3(64 * kPtWaves), 0, st, pb, (const WalkRec*)b_rec.p,
+        hipLaunchKernelGGL(k_points_alone, dim3(1), dim3(64 * kPtWaves), image_bits_bytes(n), st, pb, (const WalkRec*)b_rec.p,
                            (const AccEntry*)b_acc.p, b_pt.as<PointRec>(), b_has.as<int32_t>(), b_vis.as<int32_t>());
         PM_HIP(hipGetLastError());
         Alone a;
@@ -1940,9 +1966,9 @@ PM_API pm_status pm_fusion_run(pm_engine* e, const pm_fusion_options* o, int32_t
       if (nt > 0) {
         Flow fa = f;
         fa.n_tickets = nt;
-        hipLaunchKernelGGL(k_points, dim3((nt + kPtWaves - 1) / kPtWaves), dim3(64 * kPtWaves), 0, st,
+        hipLaunchKernelGGL(k_points, dim3((nt + kPtWaves - 1) / kPtWaves), dim3(64 * kPtWaves), image_bits_bytes(n), st,
                            (const FusImgDev*)d_tab.p, prm, (int32_t)w0, g, fa, w_pts.as<PointRec>(),
-                           w_has.as<int32_t>(), w_visp.as<int32_t>(), w_kept.as<unsigned long long>());
+                           w_has.as<int32_t>(), w_visp.as<int32_t>());
         scan(w_has.as<const int32_t>(), w_rank.as<int32_t>(), m, w_sums.as<int32_t>(), w_total.as<int32_t>(), st);
         hipLaunchKernelGGL(k_gather_points, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, st,
                            (const PointRec*)w_pts.p, (const int32_t*)w_has.p, (const int32_t*)w_rank.p, m,
