@@ -315,6 +315,9 @@ pm_status pm_engine_set_tuning(pm_engine* engine, int32_t phase, const pm_option
                                const pm_tuning* tuning);
 pm_status pm_engine_get_tuning(pm_engine* engine, int32_t phase, const pm_options* options, int32_t num_src,
                                pm_tuning* out);
+/* Columns and rows of the tiles that the view's last planned launches of the
+ * phase use; 0 before its first run and for a phase it has not. */
+pm_status pm_problem_get_tile(const pm_problem* problem, int32_t phase, int32_t* width, int32_t* height);
 /* Time every shape on this view's sweep and local-optimisation kernels and
  * keep the fastest in the engine for the view's classes.  Runs the view's
  * init and a few sweeps, so its maps are undefined until its next run. */

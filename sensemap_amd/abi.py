@@ -266,6 +266,7 @@ _SIGNATURES = {
                                        C.POINTER(pm_tuning)]),
     "pm_engine_get_tuning": (C.c_int, [C.c_void_p, C.c_int32, C.POINTER(pm_options), C.c_int32,
                                        C.POINTER(pm_tuning)]),
+    "pm_problem_get_tile": (C.c_int, [C.c_void_p, C.c_int32, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]),
     "pm_problem_autotune": (C.c_int, [C.c_void_p, C.POINTER(pm_tune_report)]),
     "pm_engine_save_tuning": (C.c_int, [C.c_void_p, C.c_char_p]),
     "pm_engine_load_tuning": (C.c_int, [C.c_void_p, C.c_char_p]),

@@ -886,7 +886,7 @@ pm_status plan_launches(const std::vector<std::pair<pm_problem*, const std::vect
     pm::LaunchCfg cfg;
     pm_tuning shape;
     std::vector<pm::LaunchEntry> e;
-    std::vector<const pm_problem*> views;  // of the entries
+    std::vector<pm_problem*> views;  // of the entries
     int tiles = 0;
     int nmax = 1;  // most sources of a view in the launch (workspace size)
     int lw = 0, lpx = pm::kTileLog2Px;
@@ -931,11 +931,17 @@ pm_status plan_launches(const std::vector<std::pair<pm_problem*, const std::vect
     }
   }
   for (Group& g : groups) {
-    long long pixels = 0;
-    for (const pm_problem* p : g.views) pixels += (long long)p->W * p->H;
-    const pm::TileShape ts = pm::tile_shape(g.kind, g.cfg, g.shape.tile_lw, pixels, g.shape.blocks_per_cu);
+    long long pixels = 0, pixel_sources = 0;
+    for (const pm_problem* p : g.views) {
+      pixels += (long long)p->W * p->H;
+      pixel_sources += (long long)p->W * p->H * p->N;
+    }
+    const pm::TileShape ts =
+        pm::tile_shape(g.kind, g.cfg, g.shape.tile_lw, pixels, pixel_sources, g.shape.blocks_per_cu);
     pm_status rs = g.number_tiles(ts.lw, ts.lpx);
     if (rs != PM_OK) return rs;
+    if (!force)
+      for (pm_problem* p : g.views) p->tile[g.kind] = {1 << ts.lw, (2 << ts.lpx) >> ts.lw};
     const int grid = pm::phase_grid(g.kind, g.cfg, g.tiles, g.shape.blocks_per_cu);
     if (grid <= 0) return fail(PM_ERR_DEVICE, "no launch configuration for a phase kernel");
     const size_t off = (plan.tables.size() + 15) & ~(size_t)15;
@@ -1237,6 +1243,15 @@ PM_API pm_status pm_engine_get_tuning(pm_engine* e, int32_t phase, const pm_opti
   pm_status rs;
   if ((rs = check_phase(phase)) != PM_OK) return rs;
   *out = shape_of(e, phase, *o, num_src);
+  return PM_OK;
+}
+
+PM_API pm_status pm_problem_get_tile(const pm_problem* p, int32_t phase, int32_t* width, int32_t* height) {
+  if (!p || !width || !height) return fail(PM_ERR_INVALID_ARG, "null argument");
+  pm_status rs;
+  if ((rs = check_phase(phase)) != PM_OK) return rs;
+  *width = p->tile[phase].w;
+  *height = p->tile[phase].h;
   return PM_OK;
 }
 

@@ -168,6 +168,9 @@ struct pm_problem {
   pm_run_stats stats{};
   size_t device_bytes = 0;
   struct pm_schedule* schedule = nullptr;
+  struct {
+    int32_t w, h;
+  } tile[PM_PHASE_MEDIAN + 1] = {};  // of the last launches planned with the view, by phase
 
   template <typename T>
   pm_status alloc(T** p, size_t count) {

@@ -320,6 +320,12 @@ class PatchMatchACMMCuda:
         abi.check(self.lib.pm_problem_write_maps(self.handle, os.fsencode(depth_path) if depth_path else None,
                                                  os.fsencode(normal_path) if normal_path else None))
 
+    def GetTile(self, phase: int):
+        """Columns and rows of the tiles the view's last launches of the phase use (pm_problem_get_tile)."""
+        w, h = C.c_int32(), C.c_int32()
+        abi.check(self.lib.pm_problem_get_tile(self.handle, int(phase), C.byref(w), C.byref(h)))
+        return w.value, h.value
+
     def Autotune(self) -> abi.pm_tune_report:
         """Time every launch shape on this view and keep the fastest in the
         engine (pm_problem_autotune); the maps are undefined until the next Run()."""
@@ -354,6 +360,7 @@ class _ProblemView:
     GetCostMap = PatchMatchACMMCuda.GetCostMap
     GetViewSelMap = PatchMatchACMMCuda.GetViewSelMap
     GetCurvatureMap = PatchMatchACMMCuda.GetCurvatureMap
+    GetTile = PatchMatchACMMCuda.GetTile
 
 
 class PatchMatchBatch:

@@ -73,3 +73,27 @@ def test_a_counted_run_gives_the_same_maps():
         e.close()
     assert not any(helpers.maps_equal(*got).values()), helpers.maps_equal(*got)
     assert np.count_nonzero(got[0]["depth"]) > 0.9 * got[0]["depth"].size
+
+
+@pytest.mark.parametrize("width,height,num_src,radius,step,sweep,local", [
+    (160, 120, 4, 5, 2, (8, 4), (8, 4)),
+    (320, 240, 1, 5, 2, (16, 8), (16, 8)),
+    # few window samples per pixel: what a tile costs once is spread over 256 pixels
+    (640, 480, 1, 5, 2, (32, 16), (32, 16)),
+    (640, 480, 4, 2, 2, (32, 16), (32, 16)),
+    (640, 480, 4, 5, 2, (16, 8), (32, 16)),
+    (640, 480, 4, 7, 1, (16, 8), (16, 8)),
+])
+def test_tiles_follow_the_work_per_pixel(width, height, num_src, radius, step, sweep, local):
+    opts = helpers.c1_options(num_iterations=4, window_radius=radius, window_step=step)
+    sc = scene.planes_scene(seed=3, width=width, height=height, f=0.8 * width, num_src=num_src)
+    e = pmm.PatchMatchACMMCuda(opts, scene.to_problem(sc))
+    assert e.GetTile(abi.PM_PHASE_SWEEP) == (0, 0)
+    print(f"[tiles] {width}x{height} sources {num_src} radius {radius}", flush=True)
+    e.Run()
+    got = maps(e)
+    tiles = e.GetTile(abi.PM_PHASE_SWEEP), e.GetTile(abi.PM_PHASE_LOCAL)
+    cpu = binding.run_view(opts, e.view)
+    e.close()
+    assert tiles == (sweep, local)
+    assert not any(helpers.maps_equal(got, cpu).values()), helpers.maps_equal(got, cpu)
