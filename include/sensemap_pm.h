@@ -283,7 +283,10 @@ void pm_batch_destroy(pm_batch* batch);
  * gives the same maps, bit for bit.  An engine keeps one shape per class:
  * phase kernel, window (radius, step), image storage, reciprocal mode and
  * source-count bucket (N <= 8, N <= 16, N > 16); classes without one use
- * tile_lw 5 and blocks_per_cu 0. */
+ * tile_lw 5 and blocks_per_cu 0.  Sweep and local-optimisation launches too
+ * small for such tiles (fewer pixels than 100 to 512 per workgroup the chip
+ * holds, by sources and window samples) have tiles of 16 x 8 or 8 x 4 pixels,
+ * whatever tile_lw; blocks_per_cu applies to them too. */
 typedef enum pm_phase {
   PM_PHASE_INIT = 0,
   PM_PHASE_SWEEP = 1,
@@ -307,7 +310,7 @@ typedef struct pm_tune_report {
   double sweep_ms_best;      /* ... chosen shape */
   double local_opt_ms_default;
   double local_opt_ms_best;
-  int32_t candidates;        /* shapes timed per kernel */
+  int32_t candidates;        /* shapes of the sweep kernel */
   int32_t reserved0;
 } pm_tune_report;
 
@@ -319,15 +322,19 @@ pm_status pm_engine_get_tuning(pm_engine* engine, int32_t phase, const pm_option
  * phase use; 0 before its first run and for a phase it has not. */
 pm_status pm_problem_get_tile(const pm_problem* problem, int32_t phase, int32_t* width, int32_t* height);
 /* Time every shape on this view's sweep and local-optimisation kernels and
- * keep the fastest in the engine for the view's classes.  Runs the view's
- * init and a few sweeps, so its maps are undefined until its next run. */
+ * keep the fastest in the engine for the view's classes.  A kernel whose
+ * launch over this view has small tiles is not tuned: the engine keeps what it
+ * holds for it, the report gives that shape, and only its time and the
+ * default's are taken.  Runs the view's init and a few sweeps, so its maps are
+ * undefined until its next run. */
 pm_status pm_problem_autotune(pm_problem* problem, pm_tune_report* report);
 /* Keep the engine's shapes in a text file, one line per class, keyed by the
  * device architecture name; loading skips lines of other architectures. */
 pm_status pm_engine_save_tuning(pm_engine* engine, const char* path);
 pm_status pm_engine_load_tuning(pm_engine* engine, const char* path);
 /* Before its first run, autotune every class of the batch that the engine
- * holds no shape for, on the class's largest view. */
+ * holds no shape for, on the class's largest views in one launch, as many as
+ * it takes for the shape to matter (none where the whole class is too small). */
 pm_status pm_batch_set_autotune(pm_batch* batch, int32_t enable);
 
 /* ---- serving loop (no counterpart in the reference) ----

@@ -1127,91 +1127,139 @@ std::vector<pm_tuning> tune_candidates(pm::PhaseKind kind, const pm_options& o) 
   return c;
 }
 
-// Time every candidate shape on one phase of view p (two rounds, the
-// minimum counts) and return the fastest.
-pm_status tune_phase(pm_problem* p, const PhaseRec& r, pm_tuning* best, double* ms_default, double* ms_best,
-                     int32_t* ncand) {
+// Whether a launch of `kind` over these views (one window class) takes the
+// shape's tiles: a small one has tiles of its own (pm::tile_shape), and all
+// shapes would be timed on the same launch.
+bool shape_matters(pm::PhaseKind kind, const std::vector<pm_problem*>& views) {
+  long long pixels = 0, pixel_sources = 0;
+  for (const pm_problem* p : views) {
+    pixels += (long long)p->W * p->H;
+    pixel_sources += (long long)p->W * p->H * p->N;
+  }
+  return pm::tile_shape(kind, cfg_of(views[0]->opt), pm::kTileLog2WDefault, pixels, pixel_sources, 0).lpx ==
+         pm::kTileLog2Px;
+}
+
+// Time the candidate shapes on one phase of the views in one launch (two
+// rounds, the minimum counts) and return the fastest.  Where the shape does
+// not matter the engine's shape stays: only the default and that one are
+// timed, and *tuned is false.
+pm_status tune_phase(const std::vector<pm_problem*>& views, const Ticks& tk, pm_tuning* best, double* ms_default,
+                     double* ms_best, int32_t* ncand, bool* tuned) {
+  pm_problem* p = views[0];
   hipStream_t s = p->engine->stream;
-  const std::vector<pm_tuning> cands = tune_candidates(r.kind, p->opt);
+  const pm::PhaseKind kind = tk[0][0][0].kind;
+  const pm_tuning def{pm::kTileLog2WDefault, 0};
+  std::vector<pm_tuning> cands = tune_candidates(kind, p->opt);
+  *ncand = (int32_t)cands.size();
+  *tuned = shape_matters(kind, views);
+  if (!*tuned) {
+    const pm_tuning held = shape_of(p->engine, kind, p->opt, p->N);
+    cands.assign(1, def);
+    if (held.tile_lw != def.tile_lw || held.blocks_per_cu != def.blocks_per_cu) cands.push_back(held);
+  }
   std::vector<double> t(cands.size(), 1e30);
-  const std::vector<pm_problem*> one{p};
-  Ticks tk(1);
-  tk[0].push_back({r});
   pm_status rs;
   for (int round = 0; round < 2; ++round) {
     for (size_t k = 0; k < cands.size(); ++k) {
       pm_schedule sch;
-      if ((rs = build_schedule(one, tk, sch, s, &cands[k])) != PM_OK) return rs;
+      if ((rs = build_schedule(views, tk, sch, s, &cands[k])) != PM_OK) return rs;
       double ms = 0.0;
       if ((rs = time_schedule(sch, s, &ms)) != PM_OK) return rs;
       t[k] = std::min(t[k], ms);
     }
   }
-  size_t kb = 0;
+  size_t kb = *tuned ? 0 : cands.size() - 1;
   *ms_default = 0.0;
   for (size_t k = 0; k < cands.size(); ++k) {
-    if (t[k] < t[kb]) kb = k;
-    if (cands[k].tile_lw == pm::kTileLog2WDefault && cands[k].blocks_per_cu == 0) *ms_default = t[k];
+    if (*tuned && t[k] < t[kb]) kb = k;
+    if (cands[k].tile_lw == def.tile_lw && cands[k].blocks_per_cu == def.blocks_per_cu) *ms_default = t[k];
   }
   *best = cands[kb];
   *ms_best = t[kb];
-  *ncand = (int32_t)cands.size();
   return PM_OK;
 }
 
-pm_status autotune(pm_problem* p, pm_tune_report* rep) {
-  pm_engine* e = p->engine;
+// Autotune on the views (one window class) advanced together, and keep the
+// shapes for the classes of the `classes` views.
+pm_status autotune(const std::vector<pm_problem*>& views, const std::vector<pm_problem*>& classes,
+                   pm_tune_report* rep) {
+  pm_engine* e = views[0]->engine;
   PM_HIP(hipSetDevice(e->device));
   hipStream_t s = e->stream;
-  const pm_options& o = p->opt;
-  const uint32_t goff = o.geom_consistency ? PM_PASS_GEOM_OFFSET : 0u;
   pm_status rs;
+  Ticks warm, sweep, local;
+  std::vector<pm_problem*> local_views;
+  for (pm_problem* p : views) {
+    const pm_options& o = p->opt;
+    const uint32_t goff = o.geom_consistency ? PM_PASS_GEOM_OFFSET : 0u;
+    warm.push_back({{{pm::kPhaseInit, 0, PM_PASS_INIT + goff, 0.0f}, {pm::kPhaseInit, 1, PM_PASS_INIT + goff, 0.0f}}});
+    for (int it = 0; it < 2; ++it)
+      for (int c = 0; c < 2; ++c)
+        warm.back().push_back({{pm::kPhaseSweep, c, PM_PASS_SWEEP(it, c) + goff, th_mc_of(o, it)}});
+    sweep.push_back({{{pm::kPhaseSweep, 0, PM_PASS_SWEEP(2, 0) + goff, th_mc_of(o, 2)}}});
+    if (!o.local_optimization) continue;
+    local_views.push_back(p);
+    local.push_back({{{pm::kPhaseLocal, 0, PM_PASS_LOCAL(3, 0) + goff, 0.0f}}});
+  }
   // a realistic state: init and two iterations of sweeps, default shapes
   {
-    Ticks warm(1);
-    warm[0] = {{{pm::kPhaseInit, 0, PM_PASS_INIT + goff, 0.0f}, {pm::kPhaseInit, 1, PM_PASS_INIT + goff, 0.0f}}};
-    for (int it = 0; it < 2; ++it)
-      for (int c = 0; c < 2; ++c) warm[0].push_back({{pm::kPhaseSweep, c, PM_PASS_SWEEP(it, c) + goff, th_mc_of(o, it)}});
-    const std::vector<pm_problem*> one{p};
-    if ((rs = prepare_views(one, false, s, true)) != PM_OK) return rs;
+    if ((rs = prepare_views(views, false, s, true)) != PM_OK) return rs;
     pm_schedule sch;
-    if ((rs = build_schedule(one, warm, sch, s, nullptr)) != PM_OK) return rs;
+    if ((rs = build_schedule(views, warm, sch, s, nullptr)) != PM_OK) return rs;
     if ((rs = launch_all(sch, s, nullptr, nullptr)) != PM_OK) return rs;
     PM_HIP(hipStreamSynchronize(s));
   }
   pm_tune_report r{};
-  const PhaseRec sw{pm::kPhaseSweep, 0, PM_PASS_SWEEP(2, 0) + goff, th_mc_of(o, 2)};
-  if ((rs = tune_phase(p, sw, &r.sweep, &r.sweep_ms_default, &r.sweep_ms_best, &r.candidates)) != PM_OK) return rs;
+  bool sweep_tuned = false, local_tuned = false;
+  if ((rs = tune_phase(views, sweep, &r.sweep, &r.sweep_ms_default, &r.sweep_ms_best, &r.candidates,
+                       &sweep_tuned)) != PM_OK)
+    return rs;
   r.local_opt = pm_tuning{pm::kTileLog2WDefault, 0};
-  if (o.local_optimization) {
-    const PhaseRec lo{pm::kPhaseLocal, 0, PM_PASS_LOCAL(3, 0) + goff, 0.0f};
+  if (!local_views.empty()) {
     int32_t nc = 0;
-    if ((rs = tune_phase(p, lo, &r.local_opt, &r.local_opt_ms_default, &r.local_opt_ms_best, &nc)) != PM_OK) return rs;
+    if ((rs = tune_phase(local_views, local, &r.local_opt, &r.local_opt_ms_default, &r.local_opt_ms_best, &nc,
+                         &local_tuned)) != PM_OK)
+      return rs;
   }
   {
     std::lock_guard<std::mutex> lk(e->tune_mu);
-    e->tuning[tune_key(pm::kPhaseSweep, o, p->N)] = r.sweep;
-    if (o.local_optimization) e->tuning[tune_key(pm::kPhaseLocal, o, p->N)] = r.local_opt;
+    for (const pm_problem* p : classes) {
+      if (sweep_tuned) e->tuning[tune_key(pm::kPhaseSweep, p->opt, p->N)] = r.sweep;
+      if (local_tuned && p->opt.local_optimization) e->tuning[tune_key(pm::kPhaseLocal, p->opt, p->N)] = r.local_opt;
+    }
   }
   if (rep) *rep = r;
   return PM_OK;
 }
 
-// Autotune, on its largest view, every sweep class of `views` the engine
-// holds no shape for.
+// Autotune the window classes of `views` that the engine holds no sweep shape
+// for, each on a launch as the run will make it: its views share launches, so
+// the largest of them are timed together, as many as it takes for the shape to
+// matter.  A class whose whole launch is too small for that has none.
 pm_status tune_batch(const std::vector<pm_problem*>& views) {
-  std::map<TuneKey, pm_problem*> largest;
+  std::map<TuneKey, std::vector<pm_problem*>> classes;
   for (pm_problem* p : views) {
-    const TuneKey k = tune_key(pm::kPhaseSweep, p->opt, p->N);
+    TuneKey k = tune_key(pm::kPhaseSweep, p->opt, p->N);
     {
       std::lock_guard<std::mutex> lk(p->engine->tune_mu);
       if (p->engine->tuning.count(k)) continue;
     }
-    auto it = largest.find(k);
-    if (it == largest.end() || (long long)p->W * p->H > (long long)it->second->W * it->second->H) largest[k] = p;
+    k.nbucket = 0;  // source counts share a launch
+    classes[k].push_back(p);
   }
-  for (auto& kv : largest) {
-    pm_status rs = autotune(kv.second, nullptr);
+  for (auto& kv : classes) {
+    std::vector<pm_problem*> by_size = kv.second, timed;
+    std::stable_sort(by_size.begin(), by_size.end(), [](const pm_problem* a, const pm_problem* b) {
+      return (long long)a->W * a->H > (long long)b->W * b->H;
+    });
+    bool matters = false;
+    for (size_t k = 0; k < by_size.size() && !matters; ++k) {
+      timed.push_back(by_size[k]);
+      matters = shape_matters(pm::kPhaseSweep, timed);
+    }
+    if (!matters) continue;
+    pm_status rs = autotune(timed, kv.second, nullptr);
     if (rs != PM_OK) return rs;
   }
   return PM_OK;
@@ -1257,7 +1305,7 @@ PM_API pm_status pm_problem_get_tile(const pm_problem* p, int32_t phase, int32_t
 
 PM_API pm_status pm_problem_autotune(pm_problem* p, pm_tune_report* report) {
   if (!p) return fail(PM_ERR_INVALID_ARG, "null problem");
-  return autotune(p, report);
+  return autotune({p}, {p}, report);
 }
 
 PM_API pm_status pm_engine_save_tuning(pm_engine* e, const char* path) {

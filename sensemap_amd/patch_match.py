@@ -328,7 +328,8 @@ class PatchMatchACMMCuda:
 
     def Autotune(self) -> abi.pm_tune_report:
         """Time every launch shape on this view and keep the fastest in the
-        engine (pm_problem_autotune); the maps are undefined until the next Run()."""
+        engine, where the view is large enough for the shape to matter
+        (pm_problem_autotune); the maps are undefined until the next Run()."""
         r = abi.pm_tune_report()
         abi.check(self.lib.pm_problem_autotune(self.handle, C.byref(r)))
         return r

@@ -186,3 +186,65 @@ def test_view_keeps_its_batch_alive():
     gc.collect()
     diff = helpers.maps_equal(grab(v), alone[1], MAPS)
     assert all(x == 0 for x in diff.values()), diff
+
+
+def saved_classes(eng, path):
+    """(phase, source-count bucket) of the shapes the engine holds."""
+    eng.save_tuning(str(path))
+    rows = [l.split() for l in path.read_text().splitlines() if not l.startswith("#")]
+    return sorted((int(r[1]), int(r[6])) for r in rows)
+
+
+def test_no_shape_is_tuned_where_it_has_no_effect(tmp_path):
+    # a launch with small tiles is the same whatever the shape: its timings tell nothing
+    opt = helpers.c1_options(num_iterations=4)
+    sc = helpers.small_planes(seed=7, width=150, height=100, f=120.0)
+    prob = scene.to_problem(sc)
+    n = len(prob.src_image_idxs)
+    eng = pmm.Engine(0)
+    e = pmm.PatchMatchACMMCuda(opt, prob, eng)
+    r = e.Autotune()
+    assert saved_classes(eng, tmp_path / "a.txt") == []
+    assert (r.sweep.tile_lw, r.sweep.blocks_per_cu) == (5, 0) and r.sweep_ms_best == r.sweep_ms_default > 0
+    # a shape given by hand stays
+    eng.set_tuning(abi.PM_PHASE_SWEEP, opt, n, 6, 2)
+    r = e.Autotune()
+    assert (r.sweep.tile_lw, r.sweep.blocks_per_cu) == (6, 2) == eng.get_tuning(abi.PM_PHASE_SWEEP, opt, n)
+    assert r.sweep_ms_best > 0 and r.sweep_ms_default > 0
+    e.close()
+    eng.close()
+    eng = pmm.Engine(0)
+    b = pmm.PatchMatchBatch([(opt, prob)] * 3, engine=eng, autotune=True)
+    b.Run()
+    assert saved_classes(eng, tmp_path / "b.txt") == []
+    b.close()
+    eng.close()
+
+
+def test_small_views_are_tuned_on_the_launch_they_share(tmp_path):
+    # 16 views, each far too small for tiles of 256 pixels, 576 000 pixels together; two source-count buckets
+    opt = helpers.c1_options(num_iterations=4)
+    few = scene.to_problem(helpers.small_planes(seed=7, width=200, height=180, f=160.0, num_src=3))
+    many = scene.to_problem(helpers.small_planes(seed=8, width=200, height=180, f=160.0, num_src=9))
+    items = [(opt, few)] * 12 + [(opt, many)] * 4
+    alone = []
+    for k in (0, 12):
+        e = pmm.PatchMatchACMMCuda(*items[k])
+        e.Run()
+        alone.append(grab(e))
+        assert e.GetTile(abi.PM_PHASE_SWEEP) == (16, 8)
+        e.close()
+    eng = pmm.Engine(0)
+    b = pmm.PatchMatchBatch(items, engine=eng, autotune=True)
+    b.Run()
+    assert saved_classes(eng, tmp_path / "c.txt") == [(p, k) for p in (abi.PM_PHASE_SWEEP, abi.PM_PHASE_LOCAL)
+                                                     for k in (0, 1)]
+    for phase in (abi.PM_PHASE_SWEEP, abi.PM_PHASE_LOCAL):
+        lw, bpc = eng.get_tuning(phase, opt, 3)
+        assert (lw, bpc) == eng.get_tuning(phase, opt, 9)
+        assert all(v.GetTile(phase) == (1 << lw, 512 >> lw) for v in b.views)
+    for k, v in enumerate(b.views):
+        diff = helpers.maps_equal(grab(v), alone[k >= 12], MAPS)
+        assert all(d == 0 for d in diff.values()), (k, diff)
+    b.close()
+    eng.close()
