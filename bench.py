@@ -16,7 +16,8 @@ step latency.
 
 roofline: the checkerboard sweep kernel, algorithmic FP32 FLOPs per launch
 (23 per bilateral-NCC window sample + 75 per (hypothesis, source) evaluation
-+ 61 per geometric term, counted in a calibration run) over its average
++ 61 per geometric term, of the evaluations the timed steps make, counted in
+a calibration run) over its average
 launch duration measured with hipEvents on the engine's stream during the
 timed steps.  cpu_baseline: the C/OpenMP transcription on a band of rows of
 the same view, photometric pass.
@@ -846,9 +847,9 @@ def main() -> int:
             geo.InitFrom(photo)
             geo.Run()
 
-    # calibration step with counting on (deterministic: same evaluations as
-    # every timed step); the atomics it adds are off for the timed steps
-    engine.set_counting(True)
+    # calibration step that counts the evaluations a timed step makes (the runs
+    # are deterministic); the atomics it adds are off for the timed steps
+    engine.set_counting(abi.PM_COUNT_MADE)
     step()
     s1 = photo.GetStats()
     s2 = None if args.only_photometric else geo.GetStats()

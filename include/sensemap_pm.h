@@ -202,8 +202,18 @@ pm_status pm_engine_create(int32_t device, pm_engine** out);
  * order, as a garbage collector finalises); the stream and the cached device
  * blocks are released with the last of them. */
 void pm_engine_destroy(pm_engine* engine);
-/* Turn on per-run counting of NCC evaluations and window samples
- * (calibration runs only; off by default). */
+/* Per-run counting of NCC evaluations, window samples and geometric terms
+ * (calibration runs only; off by default).  Both ways give the same maps.
+ * PM_COUNT_ALL (or any other value but 0 and PM_COUNT_MADE): the run makes and
+ *   counts every evaluation of the algorithm's sweep, and of a local
+ *   optimisation that drops a trial once its partial sum rules it out.
+ * PM_COUNT_MADE: the evaluations that a run without counting makes.  Its
+ *   sweep drops a refined hypothesis that can no longer win, and takes the
+ *   sources that a pixel did not select for its winner only. */
+typedef enum pm_counting {
+  PM_COUNT_ALL = 1,
+  PM_COUNT_MADE = 2
+} pm_counting;
 pm_status pm_engine_set_counting(pm_engine* engine, int32_t enable);
 
 /* Upload the view, pack poses and allocate the workspace: the

@@ -15,7 +15,8 @@ _lib = None
 
 
 class pmo_counters(C.Structure):
-    _fields_ = [("ncc_evaluations", C.c_uint64), ("ncc_samples", C.c_uint64), ("geo_evaluations", C.c_uint64)]
+    _fields_ = [(n, C.c_uint64) for n in ("ncc_evaluations", "ncc_samples", "geo_evaluations", "spare_ncc_evaluations",
+                                          "spare_ncc_samples", "spare_geo_evaluations")]
 
 
 def build() -> str:
@@ -189,7 +190,8 @@ def set_cost_fp64(on: bool) -> None:
 
 def run_view(options, view, row_begin=0, row_end=0, threads=0, count=False):
     """Run the transcription on a sensemap_amd.patch_match.ViewDesc; returns a
-    dict of depth, normal, conf, cost, view_sel (and counters if count; and
+    dict of depth, normal, conf, cost, view_sel (and if count the counters, of
+    all evaluations and of those the result needs; and
     curvature, 2 x H x W, when the options ask for the curvature map)."""
     lib = load()
     out, o = _outputs(view, options)
@@ -201,6 +203,8 @@ def run_view(options, view, row_begin=0, row_end=0, threads=0, count=False):
         raise RuntimeError("pmo_run_view failed")
     if count:
         out["counters"] = (cnt.ncc_evaluations, cnt.ncc_samples, cnt.geo_evaluations)
+        out["needed"] = (cnt.ncc_evaluations - cnt.spare_ncc_evaluations, cnt.ncc_samples - cnt.spare_ncc_samples,
+                         cnt.geo_evaluations - cnt.spare_geo_evaluations)
     return out
 
 

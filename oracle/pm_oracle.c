@@ -974,6 +974,36 @@ int pmo_select_views(const pm_options* opt, float th_mc, int nh, int N, const fl
   return best < 0 ? 0 : best;
 }
 
+/* Counts of a pixel's refinement: all of them, and the ones to spare
+ * (pmo_counters).  Dropping a hypothesis needs costs that are finite and >= 0,
+ * so that partial sums never decrease and a zero weight removes a source. */
+static void count_refinement(const pm_options* opt, int N, pmo_counters of[5][PM_MAX_NUM_SRC],
+                             float RM[5][PM_MAX_NUM_SRC], const float* wts, uint32_t sel, float best_cost, int winner,
+                             pmo_counters* cnt) {
+  const float reg = opt->geom_consistency_regularizer, most = opt->geom_consistency_max_cost;
+  const int bounded = !opt->geom_consistency || (reg >= 0.0f && most >= 0.0f && reg * most < 1e30f);
+  for (int k = 1; k < 5; ++k) {
+    float sum = 0.0f;
+    int dropped = 0;
+    for (int i = 0; i < N; ++i) {
+      const int selected = (int)((sel >> i) & 1u);
+      const int needed = !bounded || (selected ? !dropped : k == winner);
+      if (selected && !dropped) {
+        sum = sum + wts[i] * RM[k][i];
+        dropped = sum > best_cost;
+      }
+      const pmo_counters* c = &of[k][i];
+      __atomic_fetch_add(&cnt->ncc_evaluations, c->ncc_evaluations, __ATOMIC_RELAXED);
+      __atomic_fetch_add(&cnt->ncc_samples, c->ncc_samples, __ATOMIC_RELAXED);
+      __atomic_fetch_add(&cnt->geo_evaluations, c->geo_evaluations, __ATOMIC_RELAXED);
+      if (needed) continue;
+      __atomic_fetch_add(&cnt->spare_ncc_evaluations, c->ncc_evaluations, __ATOMIC_RELAXED);
+      __atomic_fetch_add(&cnt->spare_ncc_samples, c->ncc_samples, __ATOMIC_RELAXED);
+      __atomic_fetch_add(&cnt->spare_geo_evaluations, c->geo_evaluations, __ATOMIC_RELAXED);
+    }
+  }
+}
+
 static void sweep_pixel(const pass_ctx* x, int row, int col) {
   const pm_options* opt = x->opt;
   const pmo_view* v = x->v;
@@ -1031,8 +1061,11 @@ static void sweep_pixel(const pass_ctx* x, int row, int col) {
     RM[0][i] = M[best][i];
     rc[0] = rc[0] + wts[i] * RM[0][i];
   }
+  pmo_counters of[5][PM_MAX_NUM_SRC]; /* one evaluation's counts each */
+  if (x->cnt) memset(of, 0, sizeof(of));
   for (int k = 1; k < 5; ++k) {
-    for (int i = 0; i < N; ++i) RM[k][i] = mv_cost(opt, v, row, col, &ref[k], np, i, v->refK, x->cnt);
+    for (int i = 0; i < N; ++i)
+      RM[k][i] = mv_cost(opt, v, row, col, &ref[k], np, i, v->refK, x->cnt ? &of[k][i] : NULL);
   }
   for (int k = 1; k < 5; ++k) {
     float c = 0.0f;
@@ -1047,6 +1080,7 @@ static void sweep_pixel(const pass_ctx* x, int row, int col) {
       b2 = k;
     }
   }
+  if (x->cnt) count_refinement(opt, N, of, RM, wts, sel, rc[0], b2, x->cnt);
   if (b2 < 0) return;
   st->conf[p] = rc[b2];
   st->depth[p] = ref[b2].d;

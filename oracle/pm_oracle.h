@@ -108,6 +108,13 @@ typedef struct pmo_counters {
   uint64_t ncc_evaluations;
   uint64_t ncc_samples;
   uint64_t geo_evaluations;
+  /* of these, the sweep's refinement evaluations that the result does not
+   * need when a hypothesis meets the selected sources in ascending order and
+   * is dropped once its partial weighted sum exceeds the best candidate's, and
+   * only the winner meets the sources not selected */
+  uint64_t spare_ncc_evaluations;
+  uint64_t spare_ncc_samples;
+  uint64_t spare_geo_evaluations;
 } pmo_counters;
 
 /* Cost precision of the runs that follow (process-wide; for the precision

@@ -24,6 +24,7 @@ STATUS_NAMES = {
 }
 PM_STORAGE_U8, PM_STORAGE_F16 = 0, 1
 PM_ACCUM_PLAIN, PM_ACCUM_COMPENSATED = 0, 1
+PM_COUNT_ALL, PM_COUNT_MADE = 1, 2
 PM_RCP_EXACT, PM_RCP_FAST = 0, 1
 
 

@@ -50,7 +50,8 @@ struct ViewDev {
   float max_ncc_matching_cost, inv_beta2;
   int32_t num_good, num_bad, num_samples, random_optimization;
   int32_t thk, init_samples, init_random, compat_lo_geo_bug;
-  int32_t accum_mode, pad_ws;
+  int32_t accum_mode;
+  int32_t count_all;        // counted runs: make every evaluation of the algorithm (PM_COUNT_ALL)
   float conf_threshold, depth_diff_threshold;
   uint64_t seed;
   const uint8_t* ref;       // W*H

@@ -384,7 +384,7 @@ PM_API void pm_engine_destroy(pm_engine* e) {
 
 PM_API pm_status pm_engine_set_counting(pm_engine* e, int32_t enable) {
   if (!e) return fail(PM_ERR_INVALID_ARG, "null engine");
-  e->counting = enable ? 1 : 0;
+  e->counting = enable == PM_COUNT_MADE ? PM_COUNT_MADE : enable ? PM_COUNT_ALL : 0;
   return PM_OK;
 }
 
@@ -1006,11 +1006,13 @@ Ticks all_ticks(const std::vector<pm_problem*>& views) {
 
 // Per-view work before the launches: counting on/off and the initial state
 // of views created with init_depth_random = 0.
-pm_status prepare_views(const std::vector<pm_problem*>& views, bool counting, hipStream_t s, bool allow_memset) {
+pm_status prepare_views(const std::vector<pm_problem*>& views, int counting, hipStream_t s, bool allow_memset) {
   for (pm_problem* p : views) {
     unsigned long long* cnt = counting ? p->counters : nullptr;
-    if (cnt != p->host.counters) {
+    const int32_t all = counting == PM_COUNT_ALL ? 1 : 0;
+    if (cnt != p->host.counters || all != p->host.count_all) {
       p->host.counters = cnt;
+      p->host.count_all = all;
       PM_HIP(hipMemcpyAsync(p->dev, &p->host, sizeof(p->host), hipMemcpyHostToDevice, s));
     }
     if (cnt && allow_memset) PM_HIP(hipMemsetAsync(cnt, 0, 6 * sizeof(unsigned long long), s));
@@ -1073,7 +1075,7 @@ pm_status run_views(pm_engine* e, const std::vector<pm_problem*>& views, pm_sche
   hipStream_t s = e->stream;
   pm_status rs;
   if (!sch.dev && (rs = build_schedule(views, all_ticks(views), sch, s)) != PM_OK) return rs;
-  if ((rs = prepare_views(views, e->counting != 0, s, true)) != PM_OK) return rs;
+  if ((rs = prepare_views(views, e->counting, s, true)) != PM_OK) return rs;
   EventTimer t;
   std::memset(st, 0, sizeof(*st));
   if ((rs = t.rec(s)) != PM_OK) return rs;
@@ -1204,7 +1206,7 @@ pm_status autotune(const std::vector<pm_problem*>& views, const std::vector<pm_p
   }
   // a realistic state: init and two iterations of sweeps, default shapes
   {
-    if ((rs = prepare_views(views, false, s, true)) != PM_OK) return rs;
+    if ((rs = prepare_views(views, 0, s, true)) != PM_OK) return rs;
     pm_schedule sch;
     if ((rs = build_schedule(views, warm, sch, s, nullptr)) != PM_OK) return rs;
     if ((rs = launch_all(sch, s, nullptr, nullptr)) != PM_OK) return rs;
@@ -1429,10 +1431,10 @@ PM_API pm_status pm_batch_run(pm_batch* b) {
   if (!b->exec) {
     if (!b->schedule.dev && (rs = build_schedule(b->views, all_ticks(b->views), b->schedule, s)) != PM_OK) return rs;
     // counters off before capture (their pointer lives in the view block)
-    if ((rs = prepare_views(b->views, false, s, false)) != PM_OK) return rs;
+    if ((rs = prepare_views(b->views, 0, s, false)) != PM_OK) return rs;
     PM_HIP(hipStreamSynchronize(s));
     PM_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    rs = prepare_views(b->views, false, s, false);
+    rs = prepare_views(b->views, 0, s, false);
     if (rs == PM_OK) rs = launch_all(b->schedule, s, nullptr, nullptr);
     hipGraph_t g = nullptr;
     const hipError_t ce = hipStreamEndCapture(s, &g);

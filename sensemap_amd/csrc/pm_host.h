@@ -138,7 +138,7 @@ struct pm_engine {
   std::atomic<int> refs{1};
   pmh::DevCache cache;
   hipStream_t stream = nullptr;
-  int counting = 0;
+  int counting = 0;  // pm_counting
   std::mutex tune_mu;
   std::map<pmh::TuneKey, pm_tuning> tuning;  // absent = default shape
   // two pinned host buffers for large copies from and to pageable caller
@@ -310,7 +310,7 @@ pm_status plan_launches(const std::vector<std::pair<pm_problem*, const std::vect
 
 pm_status build_schedule(const std::vector<pm_problem*>& views, const Ticks& ticks, pm_schedule& sch, hipStream_t s,
                          const pm_tuning* force = nullptr);
-pm_status prepare_views(const std::vector<pm_problem*>& views, bool counting, hipStream_t s, bool allow_memset);
+pm_status prepare_views(const std::vector<pm_problem*>& views, int counting, hipStream_t s, bool allow_memset);
 pm_status launch_all(const pm_schedule& sch, hipStream_t s, EventTimer* t, pm_run_stats* st);
 pm_status run_views(pm_engine* e, const std::vector<pm_problem*>& views, pm_schedule& sch, pm_run_stats* st);
 pm_status tune_batch(const std::vector<pm_problem*>& views);

@@ -1094,7 +1094,7 @@ __device__ __forceinline__ void sweep_tile(const Ctx& cx, WinLds<R_, S_>& lds, P
   K4<float>* iK = v->refInvK;
   const float vd[3] = {iK[0] * (float)col + iK[1], iK[2] * (float)row + iK[3], 1.0f};
   const float inv_view_len = 1.0f / sqrtf(vd[0] * vd[0] + vd[1] * vd[1] + vd[2] * vd[2]);
-  const bool full = v->counters != nullptr || !costs_bounded(v);  // counted runs make every evaluation
+  const bool full = v->count_all != 0 || !costs_bounded(v);
 
   // candidates: slot 0 the current hypothesis, 1 and 2 the better of the
   // 4-neighbours, 3 + g the best of direction g
@@ -1482,13 +1482,13 @@ __device__ __forceinline__ void local_opt_tile(const Ctx& cx, WinLds<R_, S_>& ld
   // non-negative regulariser) and a float sum of non-negative terms never
   // decreases, so once sum / mw >= the pixel's conf the trial cannot be
   // taken: its remaining evaluations are skipped.  The maps are those of the
-  // full evaluation; the transcription prunes the same evaluations (and a
-  // counted run takes one source a step, as it does).
+  // full evaluation; the transcription prunes the same evaluations (a run that
+  // counts the algorithm's takes one source a step, as it does).
   const float mw = (float)__popc(sel);
   const bool prune = !v->geom || v->geom_regularizer >= 0.0f;
   float sum[kLoTrials];
   const uint32_t alive = eval_selected<R_, S_, STORE, RCP, kLoTrials>(
-      v, geo, L, ws, tile, ct, spl, R, px, part, parts, 0, sel, false, v->counters != nullptr ? 1 : cx.group, sum,
+      v, geo, L, ws, tile, ct, spl, R, px, part, parts, 0, sel, false, v->count_all != 0 ? 1 : cx.group, sum,
       [](int) __attribute__((always_inline)) { return 1.0f; },
       [&](float s) __attribute__((always_inline)) { return prune && s / mw >= conf0; },
       [&](int k, int i, int q, float m) __attribute__((always_inline)) { ws.M(k, i, q) = m; }, cnt);

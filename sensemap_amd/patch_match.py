@@ -195,7 +195,9 @@ class Engine:
         abi.check(self.lib.pm_engine_create(int(device), C.byref(h)))
         self.handle = h
 
-    def set_counting(self, enable: bool) -> None:
+    def set_counting(self, enable) -> None:
+        """0 / False: off; True or abi.PM_COUNT_ALL: every evaluation of the algorithm is made and counted;
+        abi.PM_COUNT_MADE: those that a run without counting makes (pm_engine_set_counting)."""
         abi.check(self.lib.pm_engine_set_counting(self.handle, int(enable)))
 
     def set_tuning(self, phase: int, options: PatchMatchOptions, num_src: int, tile_lw: int,

@@ -60,7 +60,7 @@ def test_bitwise_alone_and_in_a_large_launch(name):
 
 
 def test_a_counted_run_gives_the_same_maps():
-    # counting makes every evaluation of the algorithm, others leave out what cannot matter
+    # PM_COUNT_ALL makes every evaluation of the algorithm, others leave out what cannot matter
     sc = helpers.small_heightfield()
     opts = helpers.c1_options(num_iterations=5, window_radius=7, window_step=1)
     got = []
@@ -97,3 +97,44 @@ def test_tiles_follow_the_work_per_pixel(width, height, num_src, radius, step, s
     e.close()
     assert tiles == (sweep, local)
     assert not any(helpers.maps_equal(got, cpu).values()), helpers.maps_equal(got, cpu)
+
+
+@pytest.mark.parametrize("options,num_src", [
+    (dict(), 5),
+    (dict(window_radius=7, window_step=1, num_samples=20, random_optimization=False), 3),
+    (dict(geom_consistency=True), 4),
+])
+def test_counts_of_a_timed_run(options, num_src):
+    opts = helpers.c1_options(num_iterations=4, **options)
+
+    def count(view, counting, blocks_per_cu):
+        engine = pmm.Engine(0)
+        for phase in (abi.PM_PHASE_SWEEP, abi.PM_PHASE_LOCAL):
+            engine.set_tuning(phase, opts, num_src, 5, blocks_per_cu)
+        engine.set_counting(counting)
+        e = pmm.PatchMatchACMMCuda(opts, view, engine=engine)
+        e.Run()
+        st, tiles = e.GetStats(), e.GetTile(abi.PM_PHASE_SWEEP)
+        got = maps(e)
+        cpu = binding.run_view(opts, e.view, count=True)
+        e.close()
+        engine.close()
+        assert not any(helpers.maps_equal(got, cpu).values()), helpers.maps_equal(got, cpu)
+        return (st.ncc_evaluations, st.ncc_samples, st.geo_evaluations), st.sweep_ncc_evaluations, tiles, cpu
+
+    # more than 512 pixels to each of a GPU's workgroups: one source a step, the fewest evaluations
+    large = scene.to_problem(scene.planes_scene(seed=4, width=450, height=310, f=360.0, num_src=num_src),
+                             with_gt_maps=opts.geom_consistency)
+    made, sweep, tiles, cpu = count(large, abi.PM_COUNT_MADE, 1)
+    print("[counts] made", made, "all", cpu["counters"], flush=True)
+    assert tiles == (32, 16)
+    assert made == cpu["needed"]
+    every, sweep_every, _, _ = count(large, abi.PM_COUNT_ALL, 1)
+    assert every == cpu["counters"] and sweep - sweep_every == made[0] - every[0] < 0
+    # several sources a step on small tiles: some more
+    small = scene.to_problem(scene.planes_scene(seed=4, width=150, height=100, f=120.0, num_src=num_src),
+                             with_gt_maps=opts.geom_consistency)
+    made, sweep, tiles, cpu = count(small, abi.PM_COUNT_MADE, 0)
+    assert tiles == (8, 4)
+    assert all(n <= m for n, m in zip(cpu["needed"], made))
+    assert sweep < count(small, abi.PM_COUNT_ALL, 0)[1]
