@@ -4,6 +4,7 @@ bit, as running that view alone; hipGraph replays equal the eager run."""
 import numpy as np
 import pytest
 
+from oracle import binding
 from sensemap_amd import abi, scene
 from sensemap_amd import patch_match as pmm
 from tests import helpers
@@ -248,3 +249,43 @@ def test_small_views_are_tuned_on_the_launch_they_share(tmp_path):
         assert all(d == 0 for d in diff.values()), (k, diff)
     b.close()
     eng.close()
+
+
+@pytest.mark.parametrize("options,num_src", [
+    (dict(), 4),
+    (dict(window_radius=7, window_step=1, image_storage=abi.PM_STORAGE_U8), 2),
+    (dict(window_radius=6, window_step=2), 3),  # a window without a kernel of its own
+    (dict(geom_consistency=True), 3),
+])
+def test_every_tile_width_of_the_large_tiles(options, num_src):
+    # with one workgroup per CU a view of more than 512 pixels per CU has tiles of 256 pixels of a
+    # colour, whose width the shape gives; odd sizes leave part tiles on both sides
+    opt = helpers.c1_options(num_iterations=4, **options)
+    sc = helpers.small_planes(seed=9, width=421, height=317, f=340.0, num_src=num_src)
+    prob = scene.to_problem(sc, with_gt_maps=opt.geom_consistency)
+    small = scene.to_problem(helpers.small_planes(seed=2, width=77, height=45, f=60.0, num_src=num_src),
+                             with_gt_maps=opt.geom_consistency)
+    e = pmm.PatchMatchACMMCuda(opt, prob)
+    want = binding.run_view(opt, e.view)
+    e.close()
+    e = pmm.PatchMatchACMMCuda(opt, small)
+    want_small = binding.run_view(opt, e.view)
+    e.close()
+    for lw in (4, 5, 6):
+        print("[shape] tile_lw", lw, options, flush=True)
+        eng = shape_engine([(opt, prob)], lw, 1)
+        e = pmm.PatchMatchACMMCuda(opt, prob, eng)
+        e.Run()
+        for phase in (abi.PM_PHASE_INIT, abi.PM_PHASE_SWEEP, abi.PM_PHASE_LOCAL):
+            assert e.GetTile(phase) == (1 << lw, 512 >> lw)
+        diff = helpers.maps_equal(grab(e), want, MAPS)
+        e.close()
+        assert all(d == 0 for d in diff.values()), (lw, diff)
+        b = pmm.PatchMatchBatch([(opt, small), (opt, prob)], engine=eng, graph=True)
+        b.Run()
+        for k, v in enumerate(b.views):
+            assert v.GetTile(abi.PM_PHASE_SWEEP) == v.GetTile(abi.PM_PHASE_LOCAL) == (1 << lw, 512 >> lw)
+            diff = helpers.maps_equal(grab(v), (want_small, want)[k], MAPS)
+            assert all(d == 0 for d in diff.values()), (lw, k, diff)
+        b.close()
+        eng.close()
