@@ -134,13 +134,13 @@ def test_grey_and_three_channel_images_equal_transcription():
 
 
 @pytest.mark.parametrize("options", [
-    dict(),                                          # a seed's walk meets a few free nodes: replayed from registers
-    dict(max_traversal_depth=4),                     # cut by depth: from the stack
-    dict(max_num_pixels=7),                          # cut by count
-    dict(max_depth_error=0.2, max_reproj_error=12.0, max_normal_error=60.0),  # more than 64 free nodes
+    dict(),
+    dict(max_traversal_depth=4),
+    dict(max_num_pixels=7),
+    dict(max_depth_error=0.2, max_reproj_error=12.0, max_normal_error=60.0),
     dict(step_size=1, min_num_pixels=2),
 ])
-@pytest.mark.parametrize("pushes", [3, 14])          # up to 10 of a node's pushes fit a lane's registers
+@pytest.mark.parametrize("pushes", [3, 14])
 def test_replays_equal_transcription(pushes, options):
     images = orbit_images(cams=15, nbr=pushes)
     if pushes > 6:
@@ -149,4 +149,45 @@ def test_replays_equal_transcription(pushes, options):
     got, want = fuse(images, StereoFusionOptions(**options)), binding.fusion(images, StereoFusionOptions(**options))
     print("[fusion] replay", pushes, options, "points", len(got["score"]), flush=True)
     assert len(want["score"]) > 0
+    same(got, want)
+
+
+def one_pose_images(n, pushes, width=12, height=10):
+    """n images of one pose, each overlapping the `pushes` after it: a pixel's walk reaches that pixel in
+    every image and no other, so a walk from the first image has n free nodes of `pushes` free pushes each."""
+    rng = np.random.default_rng(n)
+    rows, cols = np.mgrid[0:height, 0:width]
+    ims = []
+    for k in range(n):
+        depth = (10.0 * (1 + 1e-4 * rng.standard_normal((height, width)))).astype(np.float32)
+        normal = (0.01 * rng.standard_normal((3, height, width))).astype(np.float32)
+        normal[2] -= 1.0
+        normal /= np.sqrt((normal * normal).sum(0))
+        ims.append(FusionImage((100.0, (width - 1) / 2.0, 100.0, (height - 1) / 2.0), np.eye(3), np.zeros(3), depth,
+                               normal, ((17 * rows + 5 * cols + k) % 200 + 20).astype(np.uint8),
+                               [(k + 1 + s) % n for s in range(pushes)]))
+    return ims
+
+
+# A walk is replayed from registers up to 64 free nodes of up to 10 free pushes each, where no cut by depth or
+# count can happen; else from the stack.  Both sides of each of the four limits.
+@pytest.mark.parametrize("n,pushes,options,reached", [
+    (n, pushes, {}, n) for n in (2, 63, 64, 65) for pushes in (1, 9, 10, 11) if pushes < n
+] + [
+    (40, 10, dict(max_traversal_depth=41), 40),
+    (40, 10, dict(max_traversal_depth=40), 40),
+    (40, 10, dict(max_traversal_depth=3), None),
+    (40, 10, dict(max_num_pixels=40), 40),
+    (40, 10, dict(max_num_pixels=39), 39),
+    (64, 10, dict(max_traversal_depth=65, max_num_pixels=64), 64),
+    (64, 10, dict(max_traversal_depth=64, max_num_pixels=64), 64),
+])
+def test_replays_at_their_limits(n, pushes, options, reached):
+    images = one_pose_images(n, pushes)
+    o = StereoFusionOptions(**dict(dict(min_num_pixels=2, min_num_visible_images=2), **options))
+    got, want = fuse(images, o), binding.fusion(images, o)
+    print("[fusion] one pose", n, pushes, options, "points", len(got["score"]), flush=True)
+    if reached is not None:
+        # the first image's seeds, 3 pixels inside the border, come first and take every image's pixel
+        assert (np.diff(want["vis_offsets"])[:24] == reached).all()
     same(got, want)
