@@ -31,7 +31,7 @@ HIP_FLAGS = [
 
 HIP_SOURCES = ["pm_kernels.hip", "pm_engine.hip", "pm_server.hip", "pm_io.hip", "pm_cross.hip", "pm_model.hip",
                "pm_fusion.hip"]
-# extra compile flags (tuning knobs such as -DPM_SWEEP_WAVES_PER_EU=6)
+# extra compile flags (tuning knobs such as -DPM_PIPE_DEPTH=4)
 EXTRA = os.environ.get("PM_EXTRA_HIPFLAGS", "").split()
 
 

@@ -1013,7 +1013,8 @@ __device__ __forceinline__ Head load_head(const Flow& f, int ws) {
 // the records (Head) with the likely next one loaded ahead, and the statistic
 // taken off the chain: up to the masks 6700 / 5900 (of it the predecessors'
 // depths 2000 / 0), replay 9600 / 5400, after it 3100 / 3300; k_flow 201 / 165
-// ms a call at 1920x1080 with 11 views, 24.9 / 18 ms at 640x480 with 5.
+// ms a call at 1920x1080 with 11 views, 24.9 / 18 ms at 640x480 with 5, and
+// 131 / 14.4 with the wave's own sums of the counters.
 __global__ void __launch_bounds__(64) k_flow(FusParams prm, Pool g, uint32_t* mask, Flow f) {
   __shared__ __attribute__((aligned(16))) int64_t ngid[kNodeCap];
   __shared__ __attribute__((aligned(16))) int16_t nbase[kNodeCap];

@@ -599,10 +599,10 @@ __device__ __forceinline__ float propagate_depth(float d1, const float n1[3], K4
 // ---------------------------------------------------------------------------
 // workgroup set-up shared by the colour-pass kernels
 
+// Sizes of the compiled windows (R_ >= 0); see WinLds.
 template <int R_, int S_>
 struct SpSize {
-  static constexpr int kFloats = R_ >= 0 ? ((2 * R_) / S_ + 1) * ((2 * R_) / S_ + 1)
-                                         : (2 * PM_MAX_WINDOW_RADIUS + 1) * (2 * PM_MAX_WINDOW_RADIUS + 1);
+  static constexpr int kFloats = ((2 * R_) / S_ + 1) * ((2 * R_) / S_ + 1);
 };
 
 template <int R_>
@@ -610,17 +610,13 @@ struct TileSize {
   // The staged ref tile has one row pitch for every tile shape (the widest
   // tile plus the halo), so window offsets in LDS are compile-time
   // constants; rows: the tallest tile plus the halo.
-  static constexpr int kR = R_ >= 0 ? R_ : PM_MAX_WINDOW_RADIUS;
-  static constexpr int kPitch = (1 << kTileLog2WMax) + 2 * kR;
-  static constexpr int kWords = ((kTilePixels >> kTileLog2WMin) + 2 * kR) * kPitch;
+  static constexpr int kPitch = (1 << kTileLog2WMax) + 2 * R_;
+  static constexpr int kWords = ((kTilePixels >> kTileLog2WMin) + 2 * R_) * kPitch;
 };
 
-// Stage the colour table and the ref tile (zero outside the image) into
-// LDS, then map the thread to its pixel.  Returns false for threads whose
-// pixel lies outside the image (after the barrier).
 // Persistent colour-pass kernels: a launch runs at most as many workgroups
-// as the chip holds at once, and each workgroup loops claiming 32x16 tiles
-// until the launch's tiles are exhausted.  The launch's tiles are split into
+// as the chip holds at once, and each workgroup loops claiming tiles until
+// the launch's tiles are exhausted.  The launch's tiles are split into
 // 8 contiguous ranges, one per XCD (workgroups are dispatched round-robin
 // over the XCDs, so block b starts on XCD b % 8); a workgroup takes tiles
 // from its own XCD's range first, so the workgroups of one XCD cover compact
@@ -889,11 +885,11 @@ __global__ __launch_bounds__(kSweepThreads) void k_init(const LaunchTable* __res
 // consecutive pairs still read neighbouring texels, and the four waves take
 // the list in units of one source x 64 pairs.  The source is uniform across a
 // unit: its pose and texture stay in scalar registers.  Listing also leaves
-// nothing of a pixel live across a walk but what the walk reads (122 VGPRs,
+// nothing of a pixel live across a walk but what the walk reads (126 VGPRs,
 // 4 waves per SIMD; one thread per pixel took 147 and 3).
 // Run of a 1920x1080 view (10 sources, 15x15, 8 iterations): one thread per
 // pixel 464 ms, here 342 ms.  160x120 (2 sources, 11x11 step 2, 5 iterations),
-// where the four waves share 64 pixels: 2.33 against 1.15 ms.
+// where the four waves share 16 pixels (tile_shape): 2.33 against 1.02 ms.
 
 // Per-workgroup LDS beside the window's: what the pairs need of a pixel.
 struct PassLds {
@@ -902,8 +898,8 @@ struct PassLds {
   float cost[kNumRefine * kSweepThreads];     // costs of a step, [source of the step][hypothesis][pixel]
   uint32_t sel[kSweepThreads];                // selected sources
   uint32_t bits[kSweepThreads];               // valid candidates
-  float bar[kSweepThreads];                   // cost a hypothesis has to reach
-  uint32_t win[kSweepThreads];                // workspace slot of the winner | its index << 8, or kNone
+  float norm[kSweepThreads];                  // 1 / sum of the selected sources' weights
+  uint32_t win[kSweepThreads];                // workspace slot of the winner, or kNone
   uint8_t own[4][kSweepThreads];              // per wave: pixels of a source
   int count[2][4];                            // pairs per source of a step
 };
@@ -1037,8 +1033,8 @@ __device__ __forceinline__ void eval_unselected(VPtr v, const Geo& geo, PassLds&
     for (int e0 = 0; e0 < n; e0 += 64) {
       if (e0 + lane < n) {
         const int q = own[e0 + lane];
-        const float m = eval_pair<R_, S_, STORE, RCP>(v, geo, L, tile, ct, spl, R, q, ws.hyp((int)(L.win[q] & 0xffu), q),
-                                                      i, Kgeo, cnt);
+        const float m = eval_pair<R_, S_, STORE, RCP>(v, geo, L, tile, ct, spl, R, q, ws.hyp((int)L.win[q], q), i, Kgeo,
+                                                      cnt);
         int lrow, lcol;
         geo.pixel(q, lrow, lcol);
         G(v->cost)[i * plane + (geo.row0 + lrow) * W + geo.col0 + lcol] = m;
@@ -1283,11 +1279,11 @@ __device__ __forceinline__ void sweep_tile(const Ctx& cx, WinLds<R_, S_>& lds, P
       for (int i = 0; i < N; ++i) ws.Wt(i, px) = ws.RM(0, i, px) * norm;
     }
     L.sel[px] = picked;
-    L.bar[px] = norm;
+    L.norm[px] = norm;
   }
   __syncthreads();
   sel = L.sel[px];
-  norm = L.bar[px];
+  norm = L.norm[px];
   // weight of selected source i
   auto weight = [&](int i) __attribute__((always_inline)) { return once ? norm : ws.Wt(i, px); };
   int best = -1;
