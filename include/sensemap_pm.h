@@ -294,7 +294,7 @@ void pm_batch_destroy(pm_batch* batch);
  * phase kernel, window (radius, step), image storage, reciprocal mode and
  * source-count bucket (N <= 8, N <= 16, N > 16); classes without one use
  * tile_lw 5 and blocks_per_cu 0.  Sweep and local-optimisation launches too
- * small for such tiles (fewer pixels than 100 to 512 per workgroup the chip
+ * small for such tiles (fewer pixels than 80 to 512 per workgroup the chip
  * holds, by sources and window samples) have tiles of 16 x 8 or 8 x 4 pixels,
  * whatever tile_lw; blocks_per_cu applies to them too. */
 typedef enum pm_phase {

@@ -156,14 +156,16 @@ inline bool plain_phase(PhaseKind k) { return k >= kPhaseFilter; }
 // number of CUs times the workgroups one CU holds (capped by blocks_per_cu
 // when > 0), and never more than the tiles.
 int phase_grid(PhaseKind kind, const LaunchCfg& cfg, int tiles, int blocks_per_cu);
-// Tile of a launch over views of `pixels` pixels in all, pixel_sources the sum
-// of each view's pixels times its sources, whose default or tuned width is
-// 2^lw: log2 of the width and of the pixels of one colour.
+// Pixels per workgroup slot below which a launch over such views has tiles of
+// 64 pixels of a colour.
+double small_tile_line(PhaseKind kind, const LaunchCfg& cfg, int num_src, int accum_mode);
+// Tile of a launch over views of `pixels` pixels in all, `line` their mean
+// small_tile_line, whose default or tuned width is 2^lw: log2 of the width and
+// of the pixels of one colour.
 struct TileShape {
   int lw, lpx;
 };
-TileShape tile_shape(PhaseKind kind, const LaunchCfg& cfg, int lw, long long pixels, long long pixel_sources,
-                     int blocks_per_cu);
+TileShape tile_shape(PhaseKind kind, const LaunchCfg& cfg, int lw, long long pixels, double line, int blocks_per_cu);
 // Workgroups of the phase kernel one CU holds at once.
 int phase_occupancy(PhaseKind kind, const LaunchCfg& cfg);
 hipError_t launch_phase(PhaseKind kind, const LaunchCfg& cfg, const LaunchTable* table, int grid, hipStream_t s);

@@ -879,6 +879,22 @@ pm_tuning shape_of(pm_engine* e, int kind, const pm_options& o, int N) {
   return pm_tuning{pm::kTileLog2WDefault, 0};
 }
 
+// Tile of a launch over the views: the line is the mean of theirs by pixels.
+pm::TileShape launch_tile(pm::PhaseKind kind, const pm::LaunchCfg& cfg, const std::vector<pm_problem*>& views,
+                          const pm_tuning& shape) {
+  long long pixels = 0;
+  double line = 0.0;
+  if (!pm::plain_phase(kind)) {
+    for (const pm_problem* p : views) {
+      const long long px = (long long)p->W * p->H;
+      pixels += px;
+      line += (double)px * pm::small_tile_line(kind, cfg, p->N, p->opt.accum_mode);
+    }
+    line /= (double)std::max(pixels, 1ll);
+  }
+  return pm::tile_shape(kind, cfg, shape.tile_lw, pixels, line, shape.blocks_per_cu);
+}
+
 pm_status plan_launches(const std::vector<std::pair<pm_problem*, const std::vector<PhaseRec>*>>& phases,
                         TickPlan& plan, const pm_tuning* force) {
   struct Group {
@@ -931,13 +947,7 @@ pm_status plan_launches(const std::vector<std::pair<pm_problem*, const std::vect
     }
   }
   for (Group& g : groups) {
-    long long pixels = 0, pixel_sources = 0;
-    for (const pm_problem* p : g.views) {
-      pixels += (long long)p->W * p->H;
-      pixel_sources += (long long)p->W * p->H * p->N;
-    }
-    const pm::TileShape ts =
-        pm::tile_shape(g.kind, g.cfg, g.shape.tile_lw, pixels, pixel_sources, g.shape.blocks_per_cu);
+    const pm::TileShape ts = launch_tile(g.kind, g.cfg, g.views, g.shape);
     pm_status rs = g.number_tiles(ts.lw, ts.lpx);
     if (rs != PM_OK) return rs;
     if (!force)
@@ -1133,13 +1143,7 @@ std::vector<pm_tuning> tune_candidates(pm::PhaseKind kind, const pm_options& o) 
 // shape's tiles: a small one has tiles of its own (pm::tile_shape), and all
 // shapes would be timed on the same launch.
 bool shape_matters(pm::PhaseKind kind, const std::vector<pm_problem*>& views) {
-  long long pixels = 0, pixel_sources = 0;
-  for (const pm_problem* p : views) {
-    pixels += (long long)p->W * p->H;
-    pixel_sources += (long long)p->W * p->H * p->N;
-  }
-  return pm::tile_shape(kind, cfg_of(views[0]->opt), pm::kTileLog2WDefault, pixels, pixel_sources, 0).lpx ==
-         pm::kTileLog2Px;
+  return launch_tile(kind, cfg_of(views[0]->opt), views, pm_tuning{pm::kTileLog2WDefault, 0}).lpx == pm::kTileLog2Px;
 }
 
 // Time the candidate shapes on one phase of the views in one launch (two

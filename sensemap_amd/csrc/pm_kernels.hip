@@ -2148,24 +2148,34 @@ int phase_grid(PhaseKind kind, const LaunchCfg& cfg, int tiles, int blocks_per_c
 //   96x64     4.22 / 1.79 / 1.25     160x120 (2 sources)  2.26 / 1.27 / 1.15
 //   240x160   4.50 / 2.33 / 2.87     640x480              6.58 / 6.25 / 12.9
 //   1021x767  23.0 / 24.6            1920x1080 geometric  78.1 / 78.2
+//
 // What a tile costs once weighs the more the less its pixels' walks take, so
-// the line between 256 and 64 pixels falls with the work per pixel: sources
-// times window samples, an evaluation's set-up counted as 20 samples.  Pixels
-// at which the two take the same time, against that work (11 window and source
-// counts of 9..121 samples and 1..6 sources, 1024 slots):
-//   sweep  work  29  58  87  112  168  224      local   29  58  87  116  224
-//   pixels, k   158 215 252  285  420  484             119 131 143  160  195
-// Four iterations of a view, tiles of 256 / 64 pixels: 640x480, 1 source, 11x11
-// step 2: 1.47 / 1.99 ms; 800x600, 1 source, 5x5 step 2: 1.38 / 2.80.
-TileShape tile_shape(PhaseKind kind, const LaunchCfg& cfg, int lw, long long pixels, long long pixel_sources,
-                     int blocks_per_cu) {
-  if (pixels > 0 && (kind == kPhaseSweep || kind == kPhaseLocal)) {
+// the line between 256 and 64 pixels falls with the sources and the window
+// samples of a pixel.  Thousands of pixels at which the two take the same time
+// (1024 slots; 11x11 step 2 has 36 samples, 15x15 step 2 64, 11x11 121):
+//   sources            1                2            4
+//   samples       36   64  121    36   64  121    36   64
+//   sweep        175  224  485   285  347  490   486 >520
+//   local opt.   121  128  148   146  186  330   197  323
+// Compensated moments weigh about three samples.  The lines are fitted to 756
+// views (350x262 to 832x624, 1 to 9 sources, 16 to 225 samples; u8, f16,
+// compensated, geometric), where a run takes at most 3% more than with 64
+// pixels everywhere below 512 a slot, and 4% less on average.  Four iterations,
+// 256 / 64 pixels: 640x480, 1 source, 36 samples 1.47 / 1.99 ms; 800x600, 1
+// source, 9 samples 1.38 / 2.80.
+double small_tile_line(PhaseKind kind, const LaunchCfg& cfg, int num_src, int accum_mode) {
+  const int n = 2 * cfg.radius / cfg.step + 1;
+  const double samples = (double)(n * n) * (accum_mode == PM_ACCUM_COMPENSATED ? 3.0 : 1.0);
+  const double line = kind == kPhaseSweep ? 80.0 + 1.7 * num_src * (samples + 20.0) + 0.6 * samples
+                                          : 110.0 + 0.8 * num_src * samples;
+  return line < 512.0 ? line : 512.0;
+}
+
+TileShape tile_shape(PhaseKind kind, const LaunchCfg& cfg, int lw, long long pixels, double line, int blocks_per_cu) {
+  if (kind == kPhaseSweep || kind == kPhaseLocal) {
     const long long slots = phase_grid(kind, cfg, INT32_MAX, blocks_per_cu);
-    const int n = 2 * cfg.radius / cfg.step + 1;
-    const double work = (double)pixel_sources / (double)pixels * (n * n + 20);
-    const double line = kind == kPhaseSweep ? 100.0 + 1.33 * work : 90.0 + 0.6 * work;  // pixels per slot
     if (pixels < slots / 4 * 128) return TileShape{3, 4};
-    if ((double)pixels < (double)slots * (line < 512.0 ? line : 512.0)) return TileShape{4, 6};
+    if ((double)pixels < (double)slots * line) return TileShape{4, 6};
   }
   return TileShape{lw, kTileLog2Px};
 }

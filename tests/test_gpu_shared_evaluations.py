@@ -82,6 +82,7 @@ def test_a_counted_run_gives_the_same_maps():
     (640, 480, 1, 5, 2, (32, 16), (32, 16)),
     (640, 480, 4, 2, 2, (32, 16), (32, 16)),
     (640, 480, 4, 5, 2, (16, 8), (32, 16)),
+    (600, 450, 1, 7, 1, (16, 8), (16, 8)),
     (640, 480, 4, 7, 1, (16, 8), (16, 8)),
 ])
 def test_tiles_follow_the_work_per_pixel(width, height, num_src, radius, step, sweep, local):
