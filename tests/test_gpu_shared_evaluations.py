@@ -45,16 +45,18 @@ def test_bitwise_alone_and_in_a_large_launch(name):
     e.Run()
     alone = maps(e)
     cpu = binding.run_view(opts, e.view)
+    assert e.GetTile(abi.PM_PHASE_SWEEP) == e.GetTile(abi.PM_PHASE_LOCAL) == (8, 4)
     e.close()
     assert not any(helpers.maps_equal(alone, cpu).values()), helpers.maps_equal(alone, cpu)
     # alone it runs on tiles of 16 pixels; beside a larger view on tiles of 64, and beside one of more
     # tiles than the chip has workgroup slots on tiles of 256
-    for width, height in ((480, 320), (1600, 800)):
+    for width, height, tile in ((480, 320, (16, 8)), (1600, 800, (32, 16))):
         big = scene.planes_scene(seed=7, width=width, height=height, f=900.0, num_src=2)
         rest = dict(options, geom_consistency=False, num_samples=15)
         b = pmm.PatchMatchBatch([(opts, prob), (helpers.c1_options(num_iterations=4, **rest), scene.to_problem(big))])
         b.Run()
         together = maps(b.views[0])
+        assert b.views[0].GetTile(abi.PM_PHASE_SWEEP) == tile
         b.close()
         assert not any(helpers.maps_equal(together, alone).values()), helpers.maps_equal(together, alone)
 
